@@ -40,8 +40,11 @@ struct InstBufs {
     double *phi, *phi2;
     int *t0, *t1;
     int* ls_chg;  // closest-particle pass change flags (16)
-    float *p, *r, *z, *q, *w, *s0, *s1, *pk, *Adiag, *P, *fx, *fy, *gx_, *gy_;
+    float *p, *r, *z, *q, *w, *s0, *s1, *pk, *Adiag, *P, *fx, *fy, *G;
     uint8_t* cpl;
+    uint8_t* tile_act;  // assembly tiles with a FLUID cell
+    int2* range;        // active supergroups of each strip
+    HandRows hrows;     // boundary rows of the solves
     PcgScalars* sc;
     double *qq, *ws_part, *rmax_part;
     uint32_t *mu, *mv;
@@ -54,7 +57,6 @@ struct InstBufs {
     double* partials;
     unsigned long long* sk_handoff;  // hand-off rows of the batched solver passes
     unsigned* fa_flags;              // the batch's p/r update run flags (b_fwd_axpy_kernel)
-    unsigned long long* fa_handoff;  // the batch's hand-off rows of that launch's forward solve
 };
 
 // Workgroup -> (simulation, workgroup within it) of one batched launch.
@@ -131,12 +133,16 @@ __global__ __launch_bounds__(kBlock) void b_gravity_kernel(const InstBufs* __res
                  (float)(I.dt * I.gy), vb, nvb);
 }
 
-// PcgScalars of every simulation: zero, tolerance set (one workgroup each);
-// no member is known to be done.
-__global__ void b_pcg_init_kernel(const InstBufs* __restrict__ ins, int n, double tol, int* all_done_since) {
+// PcgScalars of every simulation: zero, tolerance set, and its strips' active
+// ranges (one workgroup each); no member is known to be done.
+__global__ __launch_bounds__(kBlock) void b_pcg_init_kernel(const InstBufs* __restrict__ ins, int n, double tol,
+                                                            int* all_done_since) {
     const int b = blockIdx.x;
     if (b == 0 && threadIdx.x == 0) *all_done_since = INT_MAX;
-    if (b >= n || threadIdx.x != 0) return;
+    if (b >= n) return;
+    strip_ranges(ins[b].geom, ins[b].tile_act, ins[b].range, threadIdx.x >> 6, kBlock / 64);
+    unset_rows(ins[b].geom, ins[b].hrows, threadIdx.x, kBlock);
+    if (threadIdx.x != 0) return;
     PcgScalars z{};
     z.tol = tol;
     *ins[b].sc = z;
@@ -147,8 +153,8 @@ __global__ __launch_bounds__(kBlock) void b_assemble_kernel(const InstBufs* __re
     if (!bmap(bm, b, vb, nvb)) return;
     const InstBufs& I = ins[b];
     // solver units, A / scaleA and rhs / scaleA (as the single path's assemble)
-    assemble_sk_body(I.geom, I.cell, I.phi, I.u, I.v, I.Adiag, I.cpl, I.r, I.pk, I.s0, I.rhs_scale,
-                     I.rmax_part, (I.flags & 8) ? 0 : 1 /* FS2D_FLAG_NO_GHOST_PRESSURE */, vb, nvb);
+    assemble_sk_body(I.geom, I.cell, I.phi, I.u, I.v, I.Adiag, I.cpl, I.r, I.pk, I.s0, I.z, I.tile_act,
+                     I.rhs_scale, I.rmax_part, (I.flags & 8) ? 0 : 1 /* FS2D_FLAG_NO_GHOST_PRESSURE */, vb, nvb);
 }
 
 // The members still iterating and their virtual workgroups, packed: member b
@@ -522,7 +528,7 @@ __global__ __launch_bounds__(kBlock) void b_pc_fill_kernel(const InstBufs* __res
 struct FactorMaker {
     const int* nparts;  // workgroups of the SK launches per simulation (the rhs partials)
     __device__ FactorOp operator()(const InstBufs& I, int b) const {
-        return FactorOp{{I.Adiag}, I.cpl, {I.P, I.fx, I.fy, I.gx_, I.gy_}, I.tau, I.sigma, I.rmax_part,
+        return FactorOp{{I.Adiag}, I.cpl, {I.P, I.fx, I.fy, I.G}, I.tau, I.sigma, I.rmax_part,
                         nparts[b], I.max_iters, I.sc, I.rhs_zero};
     }
 };
@@ -587,8 +593,10 @@ struct EikSweepMaker {
 struct FwdMaker {
     const int* nparts;
     int check;
+    int h;  // iteration (-1: the initial solve)
     __device__ FwdOp operator()(const InstBufs& I, int b) const {
-        return FwdOp{{I.r, I.P, I.fx, I.fy}, nullptr, {I.q}, I.sc, I.rmax_part, nparts[b], check};
+        return FwdOp{{I.r, I.P, I.fx, I.fy}, nullptr, {I.q}, I.hrows.set(I.geom, false, h + 1),
+                     I.hrows.set(I.geom, false, h + 2), I.sc, I.rmax_part, nparts[b], check};
     }
 };
 struct BwdMaker {
@@ -598,7 +606,8 @@ struct BwdMaker {
     __device__ BwdOp operator()(const InstBufs& I, int b) const {
         // sigma_{h+1} goes where sigma_{h-1} was: the half of parity h + 1
         double* qq = I.qq + (size_t)(((h + 1) & 1) ? I.geom.S * kLoaders : 0);
-        return BwdOp{{I.q, I.P, I.gx_, I.gy_}, nullptr, {I.z}, I.sc, qq, h + 1, nullptr, 0u, check, I.rmax_part,
+        return BwdOp{{I.q, I.P, I.G}, nullptr, {I.z}, I.hrows.set(I.geom, true, h + 1),
+                     I.hrows.set(I.geom, true, h + 2), I.sc, qq, h + 1, nullptr, 0u, check, I.rmax_part,
                      check ? nparts[b] : 0};
     }
 };
@@ -611,7 +620,8 @@ struct BwdMaker {
 // had converged before iteration h, the first workgroup advances the ticket
 // by the launch's strip count and every workgroup returns, so the epochs of
 // later launches stay as if every strip had taken its ticket.
-template <class Op, bool BACKWARD, class Maker, bool PREFETCH = true>
+// ACTIVE (the pressure solves): a strip runs its active range only.
+template <class Op, bool BACKWARD, class Maker, bool ACTIVE = false, bool PREFETCH = true>
 // With `active` (the PCG plan's flags of this iteration), a strip of a member
 // that had converged before it returns once it holds its ticket, without the
 // loads its skip test would discard: its done flag makes skip() true anyway.
@@ -626,14 +636,15 @@ __global__ __launch_bounds__(kSweepThreads) void b_sweep_kernel(const InstBufs* 
         if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(ticket, (unsigned long long)sm.total);
         return;
     }
-    const unsigned long long t = sweep_ticket(L, ticket);
+    const int2* no_range = nullptr;
+    const unsigned long long t = sweep_ticket(L, ticket, no_range, 0);
     const int gs = (int)(t % (unsigned long long)sm.total);
     const unsigned epoch = (unsigned)(t / (unsigned long long)sm.total) + 1u;
     const int b = sm.inst[gs];
     const bool idle = active && active[b] == 0;
     const InstBufs& I = ins[b];
     Op op = mk(I, b);
-    const SkCtl c{ticket, I.sk_handoff, err};
+    const SkCtl c{ticket, I.sk_handoff, err, ACTIVE ? I.range : nullptr};
     if (idle) return;
     sweep_run<Op, BACKWARD, PREFETCH>(op, I.geom, c, gs - sm.first[b], epoch, L);
 }
@@ -660,7 +671,8 @@ __global__ __launch_bounds__(kSweepThreads) void b_fwd_axpy_kernel(const InstBuf
         if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(ticket, per);
         return;
     }
-    const unsigned long long t = sweep_ticket(L, ticket);
+    const int2* no_range = nullptr;
+    const unsigned long long t = sweep_ticket(L, ticket, no_range, 0);
     const int idx = (int)(t % per);
     const unsigned epoch = (unsigned)(t / per) + 1u;
     if (idx < M) {
@@ -687,8 +699,9 @@ __global__ __launch_bounds__(kSweepThreads) void b_fwd_axpy_kernel(const InstBuf
     const int gs = idx - M;
     const int b = sm.inst[gs];
     const InstBufs& I = ins[b];
-    FwdFusedOp op{{I.r, I.P, I.fx, I.fy}, nullptr, {I.q}, I.sc, I.rmax_part, count[b], 0, I.fa_flags, I.geom, epoch};
-    const SkCtl c{ticket, I.fa_handoff, err};
+    FwdFusedOp op{{I.r, I.P, I.fx, I.fy}, nullptr, {I.q}, I.hrows.set(I.geom, false, h + 1),
+                  I.hrows.set(I.geom, false, h + 2), I.sc, I.rmax_part, count[b], 0, I.fa_flags, I.geom, epoch};
+    const SkCtl c{ticket, nullptr, err, I.range};
     sweep_run<FwdFusedOp, false, PREFETCH>(op, I.geom, c, gs - sm.first[b], epoch, L);
 }
 

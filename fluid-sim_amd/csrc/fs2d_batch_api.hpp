@@ -106,8 +106,7 @@ fs2d_status balloc(fs2d_batch* B, T** p, size_t n) {
 }
 
 // Descriptor of member s (the hand-off rows and run flags are the batch's).
-InstBufs inst_bufs(const fs2d_sim* s, unsigned long long* sk_handoff, unsigned* fa_flags,
-                   unsigned long long* fa_handoff) {
+InstBufs inst_bufs(const fs2d_sim* s, unsigned long long* sk_handoff, unsigned* fa_flags) {
     InstBufs I;
     memset(&I, 0, sizeof I);  // padding too: descriptors are compared bytewise
     I.nx = s->nx; I.ny = s->ny; I.mode = s->mode; I.flags = s->flags; I.np = s->np;
@@ -120,7 +119,8 @@ InstBufs inst_bufs(const fs2d_sim* s, unsigned long long* sk_handoff, unsigned* 
     I.u = s->u; I.v = s->v; I.u2 = s->u2; I.v2 = s->v2; I.nu = s->nu; I.nv = s->nv; I.dens = s->dens; I.dens2 = s->dens2;
     I.cell = s->cell; I.cell2 = s->cell2; I.phi = s->phi; I.phi2 = s->phi2; I.t0 = s->t0; I.t1 = s->t1; I.ls_chg = s->ls_chg;
     I.p = s->p; I.r = s->r; I.z = s->z; I.q = s->q; I.w = s->w; I.s0 = s->s[0]; I.s1 = s->s[1]; I.pk = s->pk;
-    I.Adiag = s->Adiag; I.P = s->P; I.fx = s->fx; I.fy = s->fy; I.gx_ = s->gx_; I.gy_ = s->gy_; I.cpl = s->cpl;
+    I.Adiag = s->Adiag; I.P = s->P; I.fx = s->fx; I.fy = s->fy; I.G = s->G; I.cpl = s->cpl;
+    I.tile_act = s->tile_act; I.range = s->range; I.hrows = s->hrows;
     I.sc = s->sc; I.qq = s->qq; I.ws_part = s->ws_part; I.rmax_part = s->rmax_part;
     I.mu = s->mu; I.mv = s->mv; I.fu0 = s->fu0; I.fu1 = s->fu1; I.fv0 = s->fv0; I.fv1 = s->fv1; I.fcount = s->fcount;
     I.fpos = s->fpos; I.fsrc = s->fsrc; I.fkv = s->fkv;
@@ -129,7 +129,6 @@ InstBufs inst_bufs(const fs2d_sim* s, unsigned long long* sk_handoff, unsigned* 
     I.tile_sums = s->tile_sums; I.dg = s->dg; I.partials = s->partials;
     I.sk_handoff = sk_handoff;
     I.fa_flags = fa_flags;
-    I.fa_handoff = fa_handoff;
     return I;
 }
 
@@ -251,7 +250,7 @@ fs2d_status build_maps(fs2d_batch* B) {
 fs2d_status refresh_inst(fs2d_batch* B) {
     bool changed = false, counts = false;
     for (int b = 0; b < B->n; b++) {
-        InstBufs I = inst_bufs(B->sims[b], B->h_ins[b].sk_handoff, B->h_ins[b].fa_flags, B->h_ins[b].fa_handoff);
+        InstBufs I = inst_bufs(B->sims[b], B->h_ins[b].sk_handoff, B->h_ins[b].fa_flags);
         if (memcmp(&I, &B->h_ins[b], sizeof I) != 0) {
             counts = counts || I.np != B->h_ins[b].np;
             B->h_ins[b] = I;
@@ -467,7 +466,7 @@ void bpcg_iterations(fs2d_batch* B, int h0, int h1, Fwd fwd, Bwd bwd) {
         {
             Timed t(B, K_PCG_FWD);
             blaunch(B, fwd, S, kSweepThreads, B->d_ins, B->strips, B->sk_ticket, B->werr,
-                    FwdMaker{B->m_pcg.count, 1}, (const int*)B->all_done_since, h, (const int*)B->plan.active);
+                    FwdMaker{B->m_pcg.count, 1, h}, (const int*)B->all_done_since, h, (const int*)B->plan.active);
         }
         {
             Timed t(B, K_PCG_BWD);
@@ -478,35 +477,35 @@ void bpcg_iterations(fs2d_batch* B, int h0, int h1, Fwd fwd, Bwd bwd) {
 }
 void bpcg_iterations(fs2d_batch* B, int h0, int h1) {
     if (B->sweep_prefetch)
-        bpcg_iterations(B, h0, h1, b_sweep_kernel<FwdOp, false, FwdMaker, true>,
-                        b_sweep_kernel<BwdOp, true, BwdMaker, true>);
+        bpcg_iterations(B, h0, h1, b_sweep_kernel<FwdOp, false, FwdMaker, true, true>,
+                        b_sweep_kernel<BwdOp, true, BwdMaker, true, true>);
     else
-        bpcg_iterations(B, h0, h1, b_sweep_kernel<FwdOp, false, FwdMaker, false>,
-                        b_sweep_kernel<BwdOp, true, BwdMaker, false>);
+        bpcg_iterations(B, h0, h1, b_sweep_kernel<FwdOp, false, FwdMaker, true, false>,
+                        b_sweep_kernel<BwdOp, true, BwdMaker, true, false>);
 }
 
 // Assembly, MIC(0) factor and the first preconditioner application of every
 // member (FluidSim2D.cpp:252-430).
 void bpcg_begin(fs2d_batch* B) {
-    blaunch(B, b_pcg_init_kernel, B->n, 64, B->d_ins, B->n, B->tol, B->all_done_since);
     {
         Timed t(B, K_ASSEMBLE);
         blaunch(B, b_assemble_kernel, B->g_sk, kBlock, B->d_ins, B->m_sk);
     }
+    blaunch(B, b_pcg_init_kernel, B->n, kBlock, B->d_ins, B->n, B->tol, B->all_done_since);
     const int S = B->strips.total;
     {
         Timed t(B, K_FACTOR);
-        blaunch(B, b_sweep_kernel<FactorOp, false, FactorMaker>, S, kSweepThreads, B->d_ins, B->strips,
+        blaunch(B, b_sweep_kernel<FactorOp, false, FactorMaker, true>, S, kSweepThreads, B->d_ins, B->strips,
                 B->sk_ticket, B->werr, FactorMaker{B->m_sk.count}, (const int*)nullptr, 0, (const int*)nullptr);
     }
     {
         Timed t(B, K_PCG_FWD);
-        blaunch(B, b_sweep_kernel<FwdOp, false, FwdMaker>, S, kSweepThreads, B->d_ins, B->strips, B->sk_ticket,
-                B->werr, FwdMaker{B->m_sk.count, 0}, (const int*)nullptr, 0, (const int*)nullptr);
+        blaunch(B, b_sweep_kernel<FwdOp, false, FwdMaker, true>, S, kSweepThreads, B->d_ins, B->strips, B->sk_ticket,
+                B->werr, FwdMaker{B->m_sk.count, 0, -1}, (const int*)nullptr, 0, (const int*)nullptr);
     }
     {
         Timed t(B, K_PCG_BWD);
-        blaunch(B, b_sweep_kernel<BwdOp, true, BwdMaker>, S, kSweepThreads, B->d_ins, B->strips, B->sk_ticket,
+        blaunch(B, b_sweep_kernel<BwdOp, true, BwdMaker, true>, S, kSweepThreads, B->d_ins, B->strips, B->sk_ticket,
                 B->werr, BwdMaker{-1, nullptr, 0}, (const int*)nullptr, 0, (const int*)nullptr);
     }
 }
@@ -614,7 +613,7 @@ fs2d_status bfinish(fs2d_batch* B, fs2d_status st) {
     BHIPCHK(B, hipGetLastError());
     if (B->timing) resolve_timing(B);
     for (auto* s : B->sims) s->sorted_valid = false;
-    if (*B->h_err) return bfail(B, FS2D_ERR_HANG, "a wavefront hand-off wait expired");
+    if (*B->h_err) return bfail(B, FS2D_ERR_HANG, "a wavefront hand-off wait expired (site %d)", *B->h_err);
     for (int b = 0; b < B->n; b++)
         if (B->h_status[4 * b + 2]) return bfail(B, FS2D_ERR_NAN, "member %d: advected particle position is NaN", b);
     if (st == FS2D_WARN_MAXITER) {
@@ -790,13 +789,12 @@ fs2d_status fs2d_batch_create(const fs2d_config* cfgs, int n, fs2d_batch** out) 
     for (int b = 0; b < n; b++) {
         fs2d_sim* s = B->sims[b];
         const int ns = (s->ny + 63) / 64;
-        unsigned long long *skh = nullptr, *fah = nullptr;
+        unsigned long long* skh = nullptr;
         unsigned* faf = nullptr;
         if ((st = balloc(B, &skh, (size_t)ns * sk_handoff_stride(s->nx, 3))) != FS2D_OK ||
-            (st = balloc(B, &fah, (size_t)ns * sk_handoff_stride(s->nx, FwdFusedOp::NW))) != FS2D_OK ||
             (st = balloc(B, &faf, (size_t)kMaxBlocks)) != FS2D_OK)
             return bail(st);
-        B->h_ins[b] = inst_bufs(s, skh, faf, fah);
+        B->h_ins[b] = inst_bufs(s, skh, faf);
     }
     if ((st = balloc(B, &B->d_ins, (size_t)n)) != FS2D_OK) return bail(st);
     if ((st = build_maps(B)) != FS2D_OK) return bail(st);

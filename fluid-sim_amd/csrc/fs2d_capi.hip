@@ -100,24 +100,29 @@ struct fs2d_sim {
     float* p = nullptr;
     SkGeom geom{};
     float *r = nullptr, *z = nullptr, *q = nullptr, *w = nullptr, *s[2] = {nullptr, nullptr}, *pk = nullptr;
-    float *Adiag = nullptr, *P = nullptr, *fx = nullptr, *fy = nullptr, *gx_ = nullptr, *gy_ = nullptr;
+    float *Adiag = nullptr, *P = nullptr, *fx = nullptr, *fy = nullptr, *G = nullptr;
     uint8_t* cpl = nullptr;  // coupling bits (CPL_*)
+    uint8_t* tile_act = nullptr;  // assembly tiles with a FLUID cell
+    int2* range = nullptr;        // active supergroups of each strip (strip_ranges)
+    // Whether the solves read it: not when the cells are static and every
+    // assembly tile has a FLUID cell, where reading the ranges at the head of
+    // each launch cost 2% of a 1000 x 700 step and there is nothing to skip.
+    bool use_range = true;
+    HandRows hrows{};             // boundary rows of the solves
     PcgScalars* sc = nullptr;
     PcgScalars* h_sc = nullptr;
     double *qq = nullptr, *ws_part = nullptr, *rmax_part = nullptr;
     unsigned long long* sk_ticket = nullptr;
     unsigned long long* sk_handoff = nullptr;
     // a PCG iteration as two launches: the p/r update with the forward solve
-    // (fwd_axpy_kernel: its own ticket, hand-off rows and per-run flags) and
-    // the backward solve with the next SpMV (bwd_spmv_kernel: ticket,
-    // hand-off rows, per-strip completion flags, tagged sigma words)
+    // (fwd_axpy_kernel: its own ticket and per-run flags) and the backward
+    // solve with the next SpMV (bwd_spmv_kernel: ticket, per-strip completion
+    // flags, tagged sigma words)
     bool fused_pcg = true;
     int ncu = 0;  // compute units of the device
     unsigned long long* fa_ticket = nullptr;
-    unsigned long long* fa_handoff = nullptr;
     unsigned* fa_flags = nullptr;
     unsigned long long* fb_ticket = nullptr;
-    unsigned long long* fb_handoff = nullptr;
     unsigned* fb_flags = nullptr;
     unsigned long long* sig_words = nullptr;
     // extrapolation
@@ -364,9 +369,10 @@ void diagnostics(fs2d_sim* s) {
 }
 
 template <class Op, bool B>
-void launch_sweep(fs2d_sim* s, const Op& op);
+void launch_sweep(fs2d_sim* s, const Op& op, const int2* range = nullptr);
 int sk_blocks(const fs2d_sim* s);
 int pcg_blocks(const fs2d_sim* s);
+const int2* solve_range(const fs2d_sim* s) { return s->use_range ? s->range : nullptr; }
 template <int FX, int FY>
 void launch_closest(fs2d_sim* s, int k) {
     launch_sweep<ClosestSweepOp<FX, FY>, false>(
@@ -507,12 +513,10 @@ void stage_p2g(fs2d_sim* s) {
 // applyProjection (src/FluidSim2D.cpp:252-467).  Per iteration: SpMV with the
 // s update, the p/r update, forward and backward solves; scalars travel in
 // device memory, and the host reads the stopping flag once per batch.
-SkCtl sk_ctl(fs2d_sim* s) { return SkCtl{s->sk_ticket, s->sk_handoff, s->werr}; }
-
 template <class Op, bool B>
-void launch_sweep(fs2d_sim* s, const Op& op) {
+void launch_sweep(fs2d_sim* s, const Op& op, const int2* range) {
     hipLaunchKernelGGL((sweep_kernel<Op, B>), dim3(s->geom.S), dim3(kSweepThreads), 0, s->stream, op, s->geom,
-                       sk_ctl(s));
+                       SkCtl{s->sk_ticket, s->sk_handoff, s->werr, range});
 }
 
 // Workgroups of the SK4 stencil kernels: a multiple of 8 (see xcd_loop).
@@ -547,8 +551,8 @@ double solver_scale(const fs2d_sim* s) { return s->dt > 0 ? s->dt / (s->rho * s-
 void assemble(fs2d_sim* s) {
     Timed t(s, K_ASSEMBLE);
     hipLaunchKernelGGL(assemble_sk_kernel, dim3(sk_blocks(s)), dim3(kBlock), 0, s->stream, s->geom, s->cell, s->phi,
-                       s->u, s->v, s->Adiag, s->cpl, s->r, s->pk, s->s[0], 1.0 / (s->dx * solver_scale(s)),
-                       s->rmax_part, ghost_pressure(s));
+                       s->u, s->v, s->Adiag, s->cpl, s->r, s->pk, s->s[0], s->z, s->tile_act,
+                       1.0 / (s->dx * solver_scale(s)), s->rmax_part, ghost_pressure(s));
 }
 
 // Physical workgroups of the PCG SpMV and axpy launches: their loops run the
@@ -575,12 +579,13 @@ void launch_bwd_spmv(fs2d_sim* s, int next_iter, double* sig_out, const double* 
     const int K = (g.S * kLoaders + waves - 1) / waves;
     const int nbp = pcg_blocks(s);
     const int M = std::max(8, std::min(nbp, (s->ncu > 0 ? s->ncu : 256) - g.S - K));
-    BwdFusedOp op{{s->q, s->P, s->gx_, s->gy_}, nullptr, {s->z}, s->sc, nullptr, next_iter, s->fb_flags, 0u,
+    BwdFusedOp op{{s->q, s->P, s->G}, nullptr, {s->z}, s->hrows.set(g, true, next_iter),
+                  s->hrows.set(g, true, next_iter + 1), s->sc, nullptr, next_iter, s->fb_flags, 0u,
                   check, s->rmax_part, nbp};
     FusedSpmvArgs f{s->Adiag, s->cpl,     s->z, s->q,         s_old, s_new, s->w, s->sc, sig_out, s->sig_words,
                     sig_prev, first,      s->ws_part, nbp, s->fb_flags, K, M, check, s->rmax_part};
     hipLaunchKernelGGL(bwd_spmv_kernel, dim3(K + g.S + M), dim3(kSweepThreads), 0, s->stream, op, g,
-                       SkCtl{s->fb_ticket, s->fb_handoff, s->werr}, f);
+                       SkCtl{s->fb_ticket, nullptr, s->werr, solve_range(s)}, f);
 }
 
 // The p/r update of iteration h (s' in s_new, alpha = sigma_h / w.s' with
@@ -590,15 +595,16 @@ void launch_bwd_spmv(fs2d_sim* s, int next_iter, double* sig_out, const double* 
 // (every free CU) measured slower at 2048^2 (158.6 against 154.1 us), the
 // update's burst of traffic slowing the first strips.  The stopping test of
 // iteration h runs in the next backward launch.
-void launch_fwd_axpy(fs2d_sim* s, const float* s_new, const double* sig_cur) {
+void launch_fwd_axpy(fs2d_sim* s, int h, const float* s_new, const double* sig_cur) {
     const SkGeom& g = s->geom;
     const int nbp = pcg_blocks(s);
     const int per_strip = (nbp + g.S - 1) / g.S;
     const int M = std::max(8, std::min({nbp, 2 * per_strip, (s->ncu > 0 ? s->ncu : 256) - g.S}));
-    FwdFusedOp op{{s->r, s->P, s->fx, s->fy}, nullptr, {s->q}, s->sc, s->rmax_part, nbp, 0, s->fa_flags, g, 0u};
+    FwdFusedOp op{{s->r, s->P, s->fx, s->fy}, nullptr, {s->q}, s->hrows.set(g, false, h + 1),
+                  s->hrows.set(g, false, h + 2), s->sc, s->rmax_part, nbp, 0, s->fa_flags, g, 0u};
     FusedAxpyArgs f{s->pk, s->r, s_new, s->w, s->sc, sig_cur, s->ws_part, s->rmax_part, s->fa_flags, nbp, M};
     hipLaunchKernelGGL(fwd_axpy_kernel, dim3(M + g.S), dim3(kSweepThreads), 0, s->stream, op, g,
-                       SkCtl{s->fa_ticket, s->fa_handoff, s->werr}, f);
+                       SkCtl{s->fa_ticket, nullptr, s->werr, solve_range(s)}, f);
 }
 
 // MIC(0) factor and the first preconditioner application of the PCG
@@ -607,26 +613,29 @@ void launch_fwd_axpy(fs2d_sim* s, const float* s_new, const double* sig_cur) {
 // backward solve's launch also runs iteration 0's SpMV.
 void pcg_begin(fs2d_sim* s) {
     const int nb = sk_blocks(s);
-    hipLaunchKernelGGL(pcg_init_kernel, dim3(1), dim3(64), 0, s->stream, s->sc, s->tol);
+    hipLaunchKernelGGL(pcg_init_kernel, dim3(s->geom.S), dim3(64), 0, s->stream, s->sc, s->tol, s->geom, s->tile_act,
+                       s->range, s->hrows);
     {
         Timed t(s, K_FACTOR);
         // the reference skips the solve when |rhs|_inf <= 1e-12 (:447-448); r holds rhs / scaleA
-        FactorOp op{{s->Adiag}, s->cpl, {s->P, s->fx, s->fy, s->gx_, s->gy_}, s->tau, s->sigma, s->rmax_part, nb,
+        FactorOp op{{s->Adiag}, s->cpl, {s->P, s->fx, s->fy, s->G}, s->tau, s->sigma, s->rmax_part, nb,
                     s->max_iters, s->sc, 1e-12 / solver_scale(s)};
-        launch_sweep<FactorOp, false>(s, op);
+        launch_sweep<FactorOp, false>(s, op, solve_range(s));
     }
     {
         Timed t(s, K_PCG_FWD);
-        FwdOp op{{s->r, s->P, s->fx, s->fy}, nullptr, {s->q}, s->sc, s->rmax_part, nb, 0};
-        launch_sweep<FwdOp, false>(s, op);
+        FwdOp op{{s->r, s->P, s->fx, s->fy}, nullptr, {s->q}, s->hrows.set(s->geom, false, 0),
+                 s->hrows.set(s->geom, false, 1), s->sc, s->rmax_part, nb, 0};
+        launch_sweep<FwdOp, false>(s, op, solve_range(s));
     }
     {
         Timed t(s, K_PCG_BWD);
         if (s->fused_pcg) {
             launch_bwd_spmv(s, 0, s->qq, nullptr, 1, s->s[0], s->s[1], 0);
         } else {
-            BwdOp op{{s->q, s->P, s->gx_, s->gy_}, nullptr, {s->z}, s->sc, s->qq, 0};
-            launch_sweep<BwdOp, true>(s, op);
+            BwdOp op{{s->q, s->P, s->G}, nullptr, {s->z}, s->hrows.set(s->geom, true, 0),
+                     s->hrows.set(s->geom, true, 1), s->sc, s->qq, 0};
+            launch_sweep<BwdOp, true>(s, op, solve_range(s));
         }
     }
 }
@@ -651,7 +660,7 @@ void pcg_iterations(fs2d_sim* s, int h0, int h1) {
         if (s->fused_pcg) {
             {
                 Timed t(s, K_PCG_FWD);
-                launch_fwd_axpy(s, s_new, sig_cur);
+                launch_fwd_axpy(s, h, s_new, sig_cur);
             }
             Timed t(s, K_PCG_BWD);
             launch_bwd_spmv(s, h + 1, sig_prev, sig_cur, 0, s_new, s_old, 1);
@@ -670,13 +679,15 @@ void pcg_iterations(fs2d_sim* s, int h0, int h1) {
         }
         {
             Timed t(s, K_PCG_FWD);
-            FwdOp op{{s->r, s->P, s->fx, s->fy}, nullptr, {s->q}, s->sc, s->rmax_part, nbp, 1};
-            launch_sweep<FwdOp, false>(s, op);
+            FwdOp op{{s->r, s->P, s->fx, s->fy}, nullptr, {s->q}, s->hrows.set(g, false, h + 1),
+                     s->hrows.set(g, false, h + 2), s->sc, s->rmax_part, nbp, 1};
+            launch_sweep<FwdOp, false>(s, op, solve_range(s));
         }
         {
             Timed t(s, K_PCG_BWD);
-            BwdOp op{{s->q, s->P, s->gx_, s->gy_}, nullptr, {s->z}, s->sc, sig_prev, h + 1};
-            launch_sweep<BwdOp, true>(s, op);
+            BwdOp op{{s->q, s->P, s->G}, nullptr, {s->z}, s->hrows.set(g, true, h + 1),
+                     s->hrows.set(g, true, h + 2), s->sc, sig_prev, h + 1};
+            launch_sweep<BwdOp, true>(s, op, solve_range(s));
         }
     }
 }
@@ -761,7 +772,7 @@ fs2d_status finish(fs2d_sim* s, fs2d_status st) {
     HIPCHK(s, hipStreamSynchronize(s->stream));
     HIPCHK(s, hipGetLastError());
     if (s->timing) resolve_timing(s);
-    if (*s->h_err) return fail(s, FS2D_ERR_HANG, "a wavefront hand-off wait expired");
+    if (*s->h_err) return fail(s, FS2D_ERR_HANG, "a wavefront hand-off wait expired (site %d)", *s->h_err);
     if (s->h_dg->nan_flag) return fail(s, FS2D_ERR_NAN, "advected particle position is NaN");
     if (st == FS2D_WARN_MAXITER) {
         fail(s, st, "PCG: maximum iteration limit (%d) exceeded", s->max_iters);
@@ -1017,6 +1028,20 @@ static fs2d_status validate(const fs2d_config* c, char* why, size_t n) {
     return FS2D_OK;
 }
 
+// Whether every assembly tile (64 rows x 32 skewed steps) that holds cells
+// inside the walls has a FLUID one.
+static bool tiles_full(const SkGeom& g, const uint8_t* cell) {
+    const int nt = g.T4 / 8;
+    std::vector<uint8_t> inside((size_t)g.S * nt, 0), fluid((size_t)g.S * nt, 0);
+    for (int j = 1; j < g.ny - 1; j++)
+        for (int i = 1; i < g.nx - 1; i++) {
+            const size_t t = (size_t)(j >> 6) * nt + ((i + (j & 63)) >> 5);
+            inside[t] = 1;
+            fluid[t] |= cell[(size_t)j * g.nx + i] == FS2D_FLUID;
+        }
+    return inside == fluid;
+}
+
 static thread_local std::string g_create_error;
 
 fs2d_status fs2d_create(const fs2d_config* cfg, fs2d_sim** out) {
@@ -1067,9 +1092,11 @@ fs2d_status fs2d_create(const fs2d_config* cfg, fs2d_sim** out) {
     s->geom = make_geom(s->nx, s->ny);
     const size_t nS = (size_t)s->geom.size();
     s->fused_pcg = (long)nS >= kFusedPcgMinEntries;
+    s->use_range = !(s->flags & FS2D_FLAG_STATIC_CELLS) || !tiles_full(s->geom, cfg->initial_values);
     A(p, nC);
     A(r, nS); A(z, nS); A(q, nS); A(w, nS); A(s[0], nS); A(s[1], nS); A(pk, nS);
-    A(Adiag, nS); A(P, nS); A(fx, nS); A(fy, nS); A(gx_, nS); A(gy_, nS); A(cpl, nS);
+    A(Adiag, nS); A(P, nS); A(fx, nS); A(fy, nS); A(G, nS); A(cpl, nS);
+    A(tile_act, nS / 2048); A(range, (size_t)s->geom.S); A(hrows.base, HandRows::words(s->geom));
     A(sc, 1); A(qq, 2 * (size_t)s->geom.S * kLoaders); A(ws_part, kMaxBlocks); A(rmax_part, kMaxBlocks); A(sk_ticket, 1);
     A(mu, nU); A(mv, nV); A(fu0, nU); A(fv0, nV); A(fcount, 2);
     A(fu1, extra_aux_len(s->nx + 1, s->ny)); A(fv1, extra_aux_len(s->nx, s->ny + 1));
@@ -1080,9 +1107,7 @@ fs2d_status fs2d_create(const fs2d_config* cfg, fs2d_sim** out) {
     const int nstrips = (s->ny + 63) / 64;
     A(sk_handoff, (size_t)nstrips * sk_handoff_stride(s->nx, 3));
     A(fb_ticket, 1); A(fb_flags, nstrips); A(sig_words, 2 * (size_t)nstrips * kLoaders);
-    A(fb_handoff, (size_t)nstrips * sk_handoff_stride(s->nx, BwdFusedOp::NW));
     A(fa_ticket, 1); A(fa_flags, kMaxBlocks);
-    A(fa_handoff, (size_t)nstrips * sk_handoff_stride(s->nx, FwdFusedOp::NW));
 #undef A
     if (hipDeviceGetAttribute(&s->ncu, hipDeviceAttributeMultiprocessorCount, s->device) != hipSuccess) s->ncu = 0;
     e = hipHostMalloc((void**)&s->h_sc, sizeof(PcgScalars), hipHostMallocDefault);
@@ -1585,7 +1610,7 @@ constexpr long kNoallocEntries = 1L << 19;  // SK4 entries (512 x 512 cells need
 constexpr int kNoallocMaxStrips = 128;     // S * T4 <= kNoallocEntries / 256 and T4 >= 24 give S <= 85
 // hand-off words of S strips: S * (3 * (nx + 192) + 64) with nx <= 4 T4 - 64
 constexpr long kNoallocHandWords = 12L * (kNoallocEntries / 256) + 448L * kNoallocMaxStrips;
-constexpr int kNoallocFloatArrays = 13;  // r z q w s0 s1 pk Adiag P fx fy gx gy
+constexpr int kNoallocFloatArrays = 12;  // r z q w s0 s1 pk Adiag P fx fy G
 
 constexpr size_t na_align(size_t b) { return (b + 255) / 256 * 256; }
 constexpr size_t kNaFloats = na_align(sizeof(float) * kNoallocEntries);
@@ -1594,9 +1619,12 @@ constexpr size_t kNaSc = na_align(sizeof(PcgScalars));
 constexpr size_t kNaQq = na_align(sizeof(double) * 2 * kNoallocMaxStrips * kLoaders);
 constexpr size_t kNaPart = na_align(sizeof(double) * kMaxBlocks);
 constexpr size_t kNaWord = 256;
+constexpr size_t kNaTiles = na_align(kNoallocEntries / 2048);
+constexpr size_t kNaRows = na_align(sizeof(uint32_t) * 4 * (kNoallocEntries / 64));
+constexpr size_t kNaRange = na_align(sizeof(int2) * kNoallocMaxStrips);
 constexpr size_t kNaHand = na_align(sizeof(unsigned long long) * kNoallocHandWords);
 constexpr size_t kNoallocBytes =
-    kNoallocFloatArrays * kNaFloats + kNaCpl + kNaSc + kNaQq + 2 * kNaPart + 2 * kNaWord + kNaHand;
+    kNoallocFloatArrays * kNaFloats + kNaCpl + kNaSc + kNaQq + 2 * kNaPart + 2 * kNaWord + kNaTiles + kNaRange + kNaRows + kNaHand;
 
 __device__ __align__(256) unsigned char scratch[kNoallocBytes];
 
@@ -1679,7 +1707,7 @@ fs2d_status fs2d_project_noalloc(const fs2d_projection_args* a, int* iters, doub
     t.v = const_cast<float*>(a->v);
     unsigned char* q = base;
     float** fl[kNoallocFloatArrays] = {&t.r, &t.z, &t.q, &t.w, &t.s[0], &t.s[1], &t.pk,
-                                       &t.Adiag, &t.P, &t.fx, &t.fy, &t.gx_, &t.gy_};
+                                       &t.Adiag, &t.P, &t.fx, &t.fy, &t.G};
     for (float** f : fl) {
         *f = (float*)q;
         q += kNaFloats;
@@ -1691,6 +1719,9 @@ fs2d_status fs2d_project_noalloc(const fs2d_projection_args* a, int* iters, doub
     t.rmax_part = (double*)q;                    q += kNaPart;
     t.sk_ticket = (unsigned long long*)q;        q += kNaWord;
     t.werr = (int*)q;                            q += kNaWord;
+    t.tile_act = q;                              q += kNaTiles;
+    t.range = (int2*)q;                          q += kNaRange;
+    t.hrows.base = (uint32_t*)q;                 q += kNaRows;
     t.sk_handoff = (unsigned long long*)q;
     t.fused_pcg = false;  // the separate SpMV launch: no completion flags or tagged sigma in the scratch
     PcgScalars h_sc{};
@@ -1708,7 +1739,7 @@ fs2d_status fs2d_project_noalloc(const fs2d_projection_args* a, int* iters, doub
     if (e == hipSuccess) e = hipGetLastError();
     if (e != hipSuccess) return noalloc_fail(FS2D_ERR_DEVICE, "fs2d_project_noalloc: %s", hipGetErrorString(e));
     if (st < 0) return noalloc_fail(st, "fs2d_project_noalloc: %s", t.err.c_str());
-    if (h_err) return noalloc_fail(FS2D_ERR_HANG, "fs2d_project_noalloc: a wavefront hand-off wait expired");
+    if (h_err) return noalloc_fail(FS2D_ERR_HANG, "fs2d_project_noalloc: a wavefront hand-off wait expired (site %d)", h_err);
     if (iters) *iters = h_sc.iter;
     if (residual) *residual = h_sc.rhs_norm > 0 ? h_sc.r_norm / h_sc.rhs_norm : 0.0;
     if (st == FS2D_WARN_MAXITER)

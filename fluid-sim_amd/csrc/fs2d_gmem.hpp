@@ -13,6 +13,13 @@ namespace fs2d {
 
 constexpr int kSpinLimit = 1 << 16;  // polls of one memory round trip each: well under 1 s
 
+// Bounded waits that expire raise the error flag; the first one's site stays in
+// it, so the host's message can name what was waited for.
+enum WaitSite {
+    kWaitCompute = 1, kWaitLoader, kWaitPollerRing, kWaitHandoff, kWaitRuns, kWaitSigma, kWaitStrip, kWaitStrips
+};
+__device__ __forceinline__ void raise_wait(int* err, int site) { atomicCAS(err, 0, site); }
+
 // Pointers typed as global memory.  Accesses through them compile to GLOBAL
 // instructions, counted by vmcnt alone.  A pointer read from memory (the
 // batched kernels' descriptors) is otherwise generic, and FLAT accesses also

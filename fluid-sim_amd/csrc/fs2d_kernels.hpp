@@ -249,11 +249,14 @@ __device__ __forceinline__ bool sk_cell(const SkGeom& g, long e, int& i, int& j)
 // and a tile's SK4 stores fill whole cache lines (a line holds 8 rows x 4
 // steps) before they leave the L2.  Padding entries (no cell) get zeros like
 // the cells without an equation.  partials[vb]: the largest |rhs| of the
-// workgroup's tiles.
+// workgroup's tiles.  tile_act[tile]: whether the tile has a FLUID cell; the
+// solves skip the strips' ends without any (strip_ranges).  z is cleared with
+// the rest, so that the SpMV reads zeros where the solves do not write.
 __device__ __forceinline__ void assemble_sk_body(
     SkGeom g, const uint8_t* __restrict__ cell, const double* __restrict__ phi, const float* __restrict__ u,
     const float* __restrict__ v, float* __restrict__ Adiag, uint8_t* __restrict__ flags, float* __restrict__ r,
-    float* __restrict__ p, float* __restrict__ s0, double scale, double* partials, int ghost, int vb, int nvb) {
+    float* __restrict__ p, float* __restrict__ s0, float* __restrict__ z, uint8_t* __restrict__ tile_act, double scale,
+    double* partials, int ghost, int vb, int nvb) {
     constexpr double scaleA = 1.0;
     const int nx = g.nx;
     const int tiles_per_strip = g.T4 / 8;
@@ -262,6 +265,7 @@ __device__ __forceinline__ void assemble_sk_body(
     double m = 0;
     for (long tile = vb; tile < ntiles; tile += nvb) {
         const int s = (int)(tile / tiles_per_strip), t = (int)(tile % tiles_per_strip) * 32 + tt;
+        int fluid = 0;
         for (int l = rr; l < 64; l += 8) {
             const int i = t - l, j = s * 64 + l;
             const long e = (((long)s * g.T4 + (t >> 2)) * 64 + l) * 4 + (t & 3);
@@ -270,6 +274,7 @@ __device__ __forceinline__ void assemble_sk_body(
             if (i >= 0 && i < nx && j < g.ny) {
                 const long c = (long)j * nx + i;
                 if (cell[c] == FLUID) {
+                    fluid = 1;
                     const uint8_t cl = cell[c - 1], cr = cell[c + 1], cb = cell[c - nx], ct = cell[c + nx];
                     if (ghost) {
                         const double ph = phi[c];
@@ -305,9 +310,12 @@ __device__ __forceinline__ void assemble_sk_body(
             r[e] = (float)rhs;
             p[e] = 0.0f;
             s0[e] = 0.0f;
+            z[e] = 0.0f;
             const double a = fabs((double)(float)rhs);
             m = a > m ? a : m;
         }
+        fluid = __syncthreads_or(fluid);
+        if (threadIdx.x == 0) tile_act[tile] = (uint8_t)(fluid != 0);
     }
     double bm = block_max(m);
     if (threadIdx.x == 0) partials[vb] = bm;
@@ -315,8 +323,53 @@ __device__ __forceinline__ void assemble_sk_body(
 __global__ __launch_bounds__(kBlock) void assemble_sk_kernel(
     SkGeom g, const uint8_t* __restrict__ cell, const double* __restrict__ phi, const float* __restrict__ u,
     const float* __restrict__ v, float* __restrict__ Adiag, uint8_t* __restrict__ flags, float* __restrict__ r,
-    float* __restrict__ p, float* __restrict__ s0, double scale, double* partials, int ghost) {
-    assemble_sk_body(g, cell, phi, u, v, Adiag, flags, r, p, s0, scale, partials, ghost, blockIdx.x, gridDim.x);
+    float* __restrict__ p, float* __restrict__ s0, float* __restrict__ z, uint8_t* __restrict__ tile_act, double scale,
+    double* partials, int ghost) {
+    assemble_sk_body(g, cell, phi, u, v, Adiag, flags, r, p, s0, z, tile_act, scale, partials, ghost, blockIdx.x,
+                     gridDim.x);
+}
+
+// Active supergroups of strips s = first, first + stride, ... (one wave each):
+// from the first to the last tile with a FLUID cell, empty without any.
+__device__ __forceinline__ void strip_ranges(const SkGeom& g, const uint8_t* __restrict__ tile_act, int2* range,
+                                             int first, int stride) {
+    const int nt = g.T4 / 8, lane = threadIdx.x & 63;
+    for (int s = first; s < g.S; s += stride) {
+        int lo = nt, hi = 0;
+        for (int t = lane; t < nt; t += 64)
+            if (tile_act[(long)s * nt + t]) {
+                lo = min(lo, t);
+                hi = t + 1;
+            }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            lo = min(lo, __shfl_xor(lo, o, 64));
+            hi = max(hi, __shfl_xor(hi, o, 64));
+        }
+        if (lane == 0) range[s] = lo < hi ? make_int2(2 * lo, 2 * hi) : make_int2(0, 0);
+    }
+}
+// Whether 256-entry groups g0 .. g1-1 of the array hold an active one.
+__device__ __forceinline__ bool groups_active(const SkGeom& g, const int2* range, long g0, long g1) {
+    for (int s = (int)((unsigned)g0 / (unsigned)g.T4); s < g.S; s++) {
+        const long base = (long)s * g.T4;
+        if (base >= g1) break;
+        const int2 r = range[s];
+        if (max(g0, base + r.x * kSub) < min(g1, base + r.y * kSub)) return true;
+    }
+    return false;
+}
+
+// Activity of runs first, first + step, ... of nvb (64 of them from run `it`
+// on, bit k: run it + k step), the n / 256 groups split evenly over the runs;
+// every wave forms the same mask, its lanes one run each.
+__device__ __forceinline__ unsigned long long runs_active(const SkGeom& g, const int2* range, int it, int step,
+                                                          int nvb, bool from_top) {
+    if (!range) return ~0ull;
+    const long ng = g.size() >> 8;
+    const int k = it + (int)(threadIdx.x & 63) * step;
+    const int vb = from_top ? nvb - 1 - k : k;
+    return __ballot(k < nvb && groups_active(g, range, ng * vb / nvb, ng * (vb + 1) / nvb));
 }
 
 // Sum of a small partial array by one wave, broadcast to every thread of the
@@ -663,27 +716,29 @@ struct FusedSpmvArgs {
 // sigma workgroup k of K: one (strip, loader) pair per wave; the lane sums its
 // q.q over the loader's supergroups (sg = me, me + kLoaders, ... in the
 // backward solve's order), then the wave's tree, as BwdOp's loaders do.
-__device__ __forceinline__ void bwd_sigma(const SkGeom& g, const FusedSpmvArgs& f, int k, unsigned epoch) {
+__device__ __forceinline__ void bwd_sigma(const SkGeom& g, const FusedSpmvArgs& f, const int2* range, int k,
+                                          unsigned epoch) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     constexpr int kWaves = kSweepThreads / 64;
-    const int NSG = g.T4 / kSub, T = g.T4 * 4;
+    const int T = g.T4 * 4;
     for (int pr = k * kWaves + wave; pr < g.S * kLoaders; pr += f.K * kWaves) {
         const int s = pr / kLoaders, me = pr % kLoaders;
         const float* qs = f.q + (long)s * g.T4 * 256 + lane * 4;
+        const StripSpan sp = strip_span<true>(g, range, s);
         double acc = 0;
         constexpr int U = 4;  // supergroups with loads in flight together
-        for (int sg0 = me; sg0 < NSG; sg0 += U * kLoaders) {
+        for (int sg0 = sp.lo + (me + kLoaders - sp.lo % kLoaders) % kLoaders; sg0 < sp.hi; sg0 += U * kLoaders) {
             float4 v[U][kSub];
 #pragma unroll
             for (int u = 0; u < U; u++) {
                 const int sg = sg0 + u * kLoaders;
-                const int t0 = T - 16 * ((sg < NSG ? sg : NSG - 1) + 1);
+                const int t0 = T - 16 * (min(sg, sp.hi - 1) + 1);
 #pragma unroll
                 for (int j = 0; j < kSub; j++) v[u][j] = *(const float4*)(qs + (long)(t0 + 4 * j) * 64);
             }
 #pragma unroll
             for (int u = 0; u < U; u++)
-                if (sg0 + u * kLoaders < NSG)
+                if (sg0 + u * kLoaders < sp.hi)
 #pragma unroll
                     for (int j = 0; j < kSub; j++) acc += qq4(v[u][j]);
         }
@@ -699,9 +754,10 @@ __device__ __forceinline__ void bwd_sigma(const SkGeom& g, const FusedSpmvArgs& 
     }
 }
 
-// SpMV workgroup m of M.
-__device__ __forceinline__ void bwd_spmv_worker(const SkGeom& g, const FusedSpmvArgs& f, int m, unsigned epoch,
-                                                int* err) {
+// SpMV workgroup m of M.  Runs without an active group are left out: their s,
+// w, p and r stay zero, as their partials.
+__device__ __forceinline__ void bwd_spmv_worker(const SkGeom& g, const FusedSpmvArgs& f, const int2* range, int m,
+                                                unsigned epoch, int* err) {
     __shared__ int sh_bad;
     __shared__ double sh_sig;
     const int lane = threadIdx.x & 63;
@@ -723,7 +779,7 @@ __device__ __forceinline__ void bwd_spmv_worker(const SkGeom& g, const FusedSpmv
             if (__all(ok)) break;
             if (spin >= kSpinLimit || __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
                 bad = true;
-                if (lane == 0) atomicExch(err, 1);
+                if (lane == 0) raise_wait(err, kWaitSigma);
                 break;
             }
             __builtin_amdgcn_s_sleep(2);
@@ -748,10 +804,16 @@ __device__ __forceinline__ void bwd_spmv_worker(const SkGeom& g, const FusedSpmv
     // strip on either side; the strips above it finish earlier.
     const long n = g.size(), strip_sz = (long)g.T4 * 256;
     int lo_ready = g.S;  // strips lo_ready .. S-1 are known to be done
-    for (int it = m; it < f.nvb; it += f.M) {
+    unsigned long long act = 0;
+    for (int it = m, k = 0; it < f.nvb; it += f.M, k++) {
+        if ((k & 63) == 0) act = runs_active(g, range, it, f.M, f.nvb, true);
         const int vb = f.nvb - 1 - it;
         const XcdLoop xl = spmv_range(n, vb, f.nvb, (int)threadIdx.x);
         const long b0 = (n >> 8) * vb / f.nvb * 256, b1 = (n >> 8) * (vb + 1) / f.nvb * 256;
+        if (!((act >> (k & 63)) & 1)) {
+            if (threadIdx.x == 0) f.ws_partials[vb] = 0.0;
+            continue;
+        }
         const int need = b0 < b1 ? max(0, (int)(b0 / strip_sz) - 1) : g.S;
         if (need < lo_ready) {
             if (threadIdx.x < 64) {
@@ -766,7 +828,7 @@ __device__ __forceinline__ void bwd_spmv_worker(const SkGeom& g, const FusedSpmv
                     if ((unsigned)__shfl((int)v, 0, 64) == epoch) break;
                     if (spin >= kSpinLimit || __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
                         bad = true;
-                        if (lane == 0) atomicExch(err, 1);
+                        if (lane == 0) raise_wait(err, kWaitStrip);
                         break;
                     }
                     __builtin_amdgcn_s_sleep(16);
@@ -781,7 +843,7 @@ __device__ __forceinline__ void bwd_spmv_worker(const SkGeom& g, const FusedSpmv
                         if (spin >= kSpinLimit ||
                             __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
                             bad = true;
-                            if (lane == 0) atomicExch(err, 1);
+                            if (lane == 0) raise_wait(err, kWaitStrips);
                             break;
                         }
                         __builtin_amdgcn_s_sleep(8);
@@ -803,11 +865,11 @@ __device__ __forceinline__ void bwd_spmv_worker(const SkGeom& g, const FusedSpmv
 __global__ __launch_bounds__(kSweepThreads) void bwd_spmv_kernel(BwdFusedOp op, SkGeom g, SkCtl c,
                                                                  FusedSpmvArgs f) {
     __shared__ __align__(16) SweepLds<BwdFusedOp, sweep_ring<BwdFusedOp>()> L;
-    const unsigned long long ticket = sweep_ticket(L, c.ticket);
+    const unsigned long long ticket = sweep_ticket(L, c.ticket, c.range, g.S);
     const unsigned long long per = (unsigned long long)(f.K + g.S + f.M);
     const int idx = (int)(ticket % per);
     const unsigned epoch = (unsigned)(ticket / per) + 1u;
-    // sc->done is set before the launch, or by this launch's stopping test
+    // sc->done is set by an earlier launch, or by this launch's stopping test
     // (:453), which the sigma and SpMV workgroups evaluate for themselves from
     // the same partials (so they agree whether there is work) and SpMV
     // workgroup 0 records (|r|_inf; done, or the iteration count).  The
@@ -816,14 +878,17 @@ __global__ __launch_bounds__(kSweepThreads) void bwd_spmv_kernel(BwdFusedOp op, 
     const bool strip = idx >= f.K && idx < f.K + g.S;
     __shared__ int sh_done;
     if (threadIdx.x < 64) {
-        int done = f.sc->done;
+        // a value this launch itself writes does not count: strips read it while
+        // SpMV workgroup 0 may be writing it, and a strip that left would never
+        // hand its row to those that run
+        const int stamp = op.next_iter + 1, before = f.sc->done;
+        int done = before != 0 && before != stamp;
         if (!done && f.check && !strip) {
-            const double rn = f.nvb <= 64 * 32 ? wave_max_of_wide<32>(f.rmax_partials, f.nvb)
-                                               : wave_max_of(f.rmax_partials, f.nvb);
+            const double rn = wave_max_of_any(f.rmax_partials, f.nvb);
             done = rn <= f.sc->tol * f.sc->rhs_norm;
             if (idx == f.K + g.S && threadIdx.x == 0) {  // SpMV workgroup 0
                 f.sc->r_norm = rn;
-                if (done) f.sc->done = 1;
+                if (done) f.sc->done = stamp;
                 else f.sc->iter = op.next_iter;
             }
         }
@@ -832,12 +897,12 @@ __global__ __launch_bounds__(kSweepThreads) void bwd_spmv_kernel(BwdFusedOp op, 
     __syncthreads();
     if (sh_done) return;
     if (idx < f.K) {
-        bwd_sigma(g, f, idx, epoch);
+        bwd_sigma(g, f, c.range, idx, epoch);
     } else if (idx < f.K + g.S) {
         op.epoch = epoch;
         sweep_run<BwdFusedOp, true, true>(op, g, c, idx - f.K, epoch, L);
     } else {
-        bwd_spmv_worker(g, f, idx - f.K - g.S, epoch, c.err);
+        bwd_spmv_worker(g, f, c.range, idx - f.K - g.S, epoch, c.err);
     }
 }
 
@@ -938,7 +1003,8 @@ __device__ __forceinline__ void axpy_run_wave(RunBuf& B, const float4* s4, const
 // 256 threads of its first four waves on one run at a time: a run of a large
 // grid is about 540 float4s, which one wave would take in three round trips
 // (per-wave runs measured 157.2 against 150.9 us per launch at 2048^2).
-__device__ __forceinline__ void fwd_axpy_worker(const SkGeom& g, const FusedAxpyArgs& f, int m, unsigned epoch) {
+__device__ __forceinline__ void fwd_axpy_worker(const SkGeom& g, const FusedAxpyArgs& f, const int2* range, int m,
+                                                unsigned epoch) {
     float4* p4 = (float4*)f.p;
     const float4* s4 = (const float4*)f.s;
     const float4* w4 = (const float4*)f.w;
@@ -962,28 +1028,25 @@ __device__ __forceinline__ void fwd_axpy_worker(const SkGeom& g, const FusedAxpy
     long q0, q1;
     pcg_run(g.size(), m, f.nvb, q0, q1);
     if (threadIdx.x < kBlock) load(q0 + threadIdx.x, q1);
+    unsigned long long act = runs_active(g, range, m, f.M, f.nvb, false);
     // alpha = sigma / w.s as pcg_axpy_sk_kernel's block_sum_bcast forms it,
     // with every load of both sums in flight together (one memory round
     // trip: the update's first runs, and so the first strip, wait on it)
     __shared__ float sh_a;
     if (threadIdx.x < 64) {
         double sig, ws;
-        if (g.S * kLoaders <= 64 * 12 && f.nvb <= 64 * 32) {
-            wave_sum_of_wide2<12, 32>(f.sig_cur, g.S * kLoaders, f.ws_partials, f.nvb, sig, ws);
-        } else {
-            sig = wave_sum_of(f.sig_cur, g.S * kLoaders);
-            ws = wave_sum_of(f.ws_partials, f.nvb);
-        }
+        wave_sum_of_any2(f.sig_cur, g.S * kLoaders, f.ws_partials, f.nvb, sig, ws);
         if (threadIdx.x == 0) sh_a = (float)(sig / ws);
     }
     __syncthreads();
     const float a = sh_a;
     const __amdgpu_buffer_rsrc_t r_rs = __builtin_amdgcn_make_buffer_rsrc(f.r, 0, (int)(g.size() * 4), kBufferCfg);
     typedef float f4 __attribute__((ext_vector_type(4)));
-    for (int vb = m; vb < f.nvb; vb += f.M) {
+    for (int vb = m, k = 0; vb < f.nvb; vb += f.M, k++) {
+        if (k && (k & 63) == 0) act = runs_active(g, range, vb, f.M, f.nvb, false);
         pcg_run(g.size(), vb, f.nvb, q0, q1);
         float mx = 0.0f;
-        if (threadIdx.x < kBlock) {
+        if (threadIdx.x < kBlock && ((act >> (k & 63)) & 1)) {
             for (long e0 = q0 + threadIdx.x; e0 < q1; e0 += U * kBlock) {
                 if (vb != m || e0 != q0 + threadIdx.x) load(e0, q1);
 #pragma unroll
@@ -1020,7 +1083,7 @@ __device__ __forceinline__ void fwd_axpy_worker(const SkGeom& g, const FusedAxpy
 __global__ __launch_bounds__(kSweepThreads) void fwd_axpy_kernel(FwdFusedOp op, SkGeom g, SkCtl c,
                                                                  FusedAxpyArgs f) {
     __shared__ __align__(16) SweepLds<FwdFusedOp, sweep_ring<FwdFusedOp>()> L;
-    const unsigned long long ticket = sweep_ticket(L, c.ticket);
+    const unsigned long long ticket = sweep_ticket(L, c.ticket, c.range, g.S);
     const unsigned long long per = (unsigned long long)(f.M + g.S);
     const int idx = (int)(ticket % per);
     const unsigned epoch = (unsigned)(ticket / per) + 1u;
@@ -1030,15 +1093,26 @@ __global__ __launch_bounds__(kSweepThreads) void fwd_axpy_kernel(FwdFusedOp op, 
     __syncthreads();
     if (sh_done) return;
     if (idx < f.M) {
-        fwd_axpy_worker(g, f, idx, epoch);
+        fwd_axpy_worker(g, f, c.range, idx, epoch);
     } else {
         op.epoch = epoch;
         sweep_run<FwdFusedOp, false, true>(op, g, c, idx - f.M, epoch, L);
     }
 }
 
-// PcgScalars of one projection: zero, tolerance set (:424-430).
-__global__ void pcg_init_kernel(PcgScalars* sc, double tol) {
+// PcgScalars of one projection: zero, tolerance set (:424-430); and the
+// strips' active ranges from the assembly's tile flags (a wave per workgroup);
+// the first passes' boundary rows unset.
+__device__ __forceinline__ void unset_rows(const SkGeom& g, HandRows rows, int tid, int nt) {
+    const uint4 v = make_uint4(kUnset, kUnset, kUnset, kUnset);
+    uint4 *f = (uint4*)rows.set(g, false, 0), *b = (uint4*)rows.set(g, true, 0);
+    for (int k = tid; k < g.S * g.T4; k += nt) f[k] = b[k] = v;
+}
+__global__ __launch_bounds__(64) void pcg_init_kernel(PcgScalars* sc, double tol, SkGeom g,
+                                                      const uint8_t* __restrict__ tile_act, int2* range,
+                                                      HandRows rows) {
+    strip_ranges(g, tile_act, range, blockIdx.x, gridDim.x);
+    unset_rows(g, rows, blockIdx.x * 64 + threadIdx.x, gridDim.x * 64);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         PcgScalars z{};
         z.tol = tol;
@@ -2064,9 +2138,9 @@ struct ClosestSweepOp {
         x[4] = make_float4(hi[0], hi[1], hi[2], hi[3]);
     }
     __device__ void loader_done(int, int, double) const {}
-    template <bool B, bool C>
+    template <bool B, bool C, class H>
     __device__ void group(const float4 (&x)[NF], uint32_t, uint32_t (&st)[NW], const uint4 (&hb)[NW],
-                          float (&o)[NOUT][4], uint32_t (&prod)[NW][4], int t0, int s) {
+                          float (&o)[NOUT][4], uint32_t (&prod)[NW][4], int t0, int s, H) {
         const int lane = threadIdx.x & 63;
         const int b = 64 * s + lane;
         const int j = FY ? ny - 1 - b : b;
@@ -2258,9 +2332,9 @@ struct EikSweepOp {
         x[1] = in[1];
     }
     __device__ void loader_done(int, int, double) const {}
-    template <bool B, bool C>
+    template <bool B, bool C, class H>
     __device__ void group(const float4 (&x)[NF], uint32_t b4, uint32_t (&st)[NW], const uint4 (&hb)[NW],
-                          float (&o)[NOUT][4], uint32_t (&prod)[NW][4], int, int) const {
+                          float (&o)[NOUT][4], uint32_t (&prod)[NW][4], int, int, H) const {
 #pragma unroll
         for (int q = 0; q < 4; q++) {
             uint32_t nb[NW];
