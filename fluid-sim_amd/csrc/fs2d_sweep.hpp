@@ -291,8 +291,16 @@ __device__ __forceinline__ void sweep_compute(Op& op, const SkGeom& g, SweepLds<
     int row_off = 0;
     if constexpr (ROW) {
         row_rs = __builtin_amdgcn_make_buffer_rsrc(op.row + (size_t)s * T, 0, T * 4, kBufferCfg);
-        row_off = lane == prod_lane ? 0 : 0x40000000;
+        row_off = (lane == prod_lane ? 0 : 0x40000000) + 4 * (B ? T - 16 * (sp.lo + 1) : 16 * sp.lo);
     }
+    // Byte offsets of the buffer stores, advanced by a supergroup at a time: in
+    // registers, not in the instruction's scalar offset.  A 16-byte buffer store
+    // with a scalar offset still reads its data while the next instruction
+    // executes, and where that one overwrites the data, lanes 28-31 stored the
+    // new value (seen on gfx950; the compiler places the wait states only for
+    // stores without one).
+    int out_off = (int)((strip_base + (B ? T - 16 * (sp.lo + 1) : 16 * sp.lo) * 64L + lane * 4) * 4);
+    constexpr int kOutInc = B ? -4096 : 4096, kRowInc = B ? -64 : 64;
 
     struct Buf {
         float4 x[kSub][NF];
@@ -414,8 +422,7 @@ __device__ __forceinline__ void sweep_compute(Op& op, const SkGeom& g, SweepLds<
                 if (THROUGH) {
                     typedef float f4 __attribute__((ext_vector_type(4)));
                     const f4 v = {o[n][0], o[n][1], o[n][2], o[n][3]};
-                    __builtin_amdgcn_raw_buffer_store_b128(v, out_rs[n], (j * 256 + lane * 4) * 4,
-                                                           (int)((strip_base + (long)t0 * 64) * 4), kCpolSc1);
+                    __builtin_amdgcn_raw_buffer_store_b128(v, out_rs[n], out_off + j * 1024, 0, kCpolSc1);
                 } else {
                     float* base = op.out[n] + strip_base + (long)t0 * 64;  // uniform
                     *(float4*)(base + j * 256 + lane * 4) = make_float4(o[n][0], o[n][1], o[n][2], o[n][3]);
@@ -425,7 +432,7 @@ __device__ __forceinline__ void sweep_compute(Op& op, const SkGeom& g, SweepLds<
                 if (P) {
                     typedef float f4 __attribute__((ext_vector_type(4)));
                     const f4 v = {o[0][0], o[0][1], o[0][2], o[0][3]};
-                    __builtin_amdgcn_raw_buffer_store_b128(v, row_rs, row_off + 16 * j, 4 * t0, kCpolSc1);
+                    __builtin_amdgcn_raw_buffer_store_b128(v, row_rs, row_off + 16 * j, 0, kCpolSc1);
                 }
             } else if (P)
 #pragma unroll
@@ -446,6 +453,8 @@ __device__ __forceinline__ void sweep_compute(Op& op, const SkGeom& g, SweepLds<
             }
             __builtin_amdgcn_sched_barrier(0);
         }
+        if (THROUGH) out_off += kOutInc;
+        if (ROW && P) row_off += kRowInc;
         lds_st(done_v, (unsigned)sg + 1u);
         const unsigned sn1 = (unsigned)sn + 1u;
         const unsigned tv = uniform(tagv), hv = C ? uniform(hrv) : 0u;
