@@ -20,6 +20,7 @@
 #include <climits>
 
 #include "fs2d_kernels.hpp"
+#include "fs2d_pcg_loop.hpp"
 
 namespace fs2d {
 
@@ -45,6 +46,7 @@ struct InstBufs {
     uint8_t* tile_act;  // assembly tiles with a FLUID cell
     int2* range;        // active supergroups of each strip
     HandRows hrows;     // boundary rows of the solves
+    unsigned long long* loop_words;  // the one-launch solve's tagged words
     PcgScalars* sc;
     double *qq, *ws_part, *rmax_part;
     uint32_t *mu, *mv;
@@ -145,6 +147,7 @@ __global__ __launch_bounds__(kBlock) void b_pcg_init_kernel(const InstBufs* __re
     if (threadIdx.x != 0) return;
     PcgScalars z{};
     z.tol = tol;
+    z.epoch = ins[b].sc->epoch + (unsigned)ins[b].sc->iter + 4u;
     *ins[b].sc = z;
 }
 
@@ -266,12 +269,23 @@ __global__ __launch_bounds__(kBlock) void b_spmv_kernel(const InstBufs* __restri
         if (b < 0) continue;  // padding to a multiple of 8
         const int vb = k - P.first[b], nvb = count[b];
         const InstBufs& I = ins[b];
+        if (I.loop_words) continue;  // b_spmv_strip_kernel's
         const float* s_old = (h & 1) ? I.s1 : I.s0;
         float* s_new = (h & 1) ? I.s0 : I.s1;
         const SpmvPre pre = spmv_pre(I.geom, I.Adiag, I.cpl, I.z, s_old, vb, nvb);
         const float beta = I.sc->beta;  // b_pcg_plan_kernel's, as spmv_scalars forms it
         spmv_core(pre, I.geom, I.Adiag, I.cpl, I.z, s_old, s_new, I.w, beta, I.ws_part, vb);
     }
+}
+// The same for members whose single solve runs in one launch, with its order of
+// the w.s sum: a strip per workgroup.
+__global__ __launch_bounds__(kLoopThreads) void b_spmv_strip_kernel(const InstBufs* __restrict__ ins, StripMap sm,
+                                                                    int h) {
+    const int b = sm.inst[blockIdx.x];
+    const InstBufs& I = ins[b];
+    if (!I.loop_words || I.sc->done) return;
+    spmv_strip_body(I.geom, I.Adiag, I.z, (h & 1) ? I.s1 : I.s0, (h & 1) ? I.s0 : I.s1, I.w, I.sc->beta,
+                    I.ws_part, I.range, (int)blockIdx.x - sm.first[b]);
 }
 // w.s of every member still iterating, summed once per member (one wave per
 // member) in the order the single launch's axpy sums it, so that the axpy's
@@ -283,7 +297,7 @@ __global__ __launch_bounds__(64) void b_ws_reduce_kernel(const InstBufs* __restr
     if (b >= n) return;
     const InstBufs& I = ins[b];
     if (I.sc->done) return;
-    const double t = wave_sum_of(I.ws_part, nparts[b]);
+    const double t = wave_sum_of(I.ws_part, I.loop_words ? I.geom.S : nparts[b]);
     if (threadIdx.x == 0) I.sc->ws = t;
 }
 __global__ __launch_bounds__(kBlock) void b_axpy_kernel(const InstBufs* __restrict__ ins,
@@ -649,6 +663,24 @@ __global__ __launch_bounds__(kSweepThreads) void b_sweep_kernel(const InstBufs* 
     sweep_run<Op, BACKWARD, PREFETCH>(op, I.geom, c, gs - sm.first[b], epoch, L);
 }
 
+
+// The whole PCG of every member in one launch (fs2d_pcg_loop.hpp): each member
+// iterates at its own pace until it has converged, so a strip's workgroup
+// waits only for its own simulation, and a workgroup that finishes makes room
+// for the next member's.  Strips are taken in the order of the strip list.
+__global__ __launch_bounds__(kLoopThreads) void b_pcg_loop_kernel(const InstBufs* __restrict__ ins, StripMap sm,
+                                                                  unsigned long long* ticket, int* err) {
+    __shared__ __align__(16) LoopLds L;
+    __shared__ unsigned long long sh_ticket;
+    if (threadIdx.x == 0) sh_ticket = atomicAdd(ticket, 1ull);
+    __syncthreads();
+    const int gs = (int)uniform((unsigned)(sh_ticket % (unsigned long long)sm.total));
+    const int b = sm.inst[gs];
+    const InstBufs& I = ins[b];
+    const LoopArgs A{I.geom, I.Adiag, I.r, I.pk, I.s0,    I.s1,    I.w,          I.z,        I.q, I.P,
+                     I.fx,   I.fy,    I.G,   I.sc, I.range, I.hrows, I.loop_words, I.max_iters};
+    pcg_loop_strip(A, gs - sm.first[b], L, err);
+}
 
 // Iteration h's p/r update and forward solves of every member in one launch,
 // as fwd_axpy_kernel does for one simulation: the waves of M workgroups run

@@ -46,6 +46,9 @@ struct fs2d_batch {
     // hide in (107.4 against 103.6 ms per step); the autotuner tries both.
     bool fused_pcg = false;
     unsigned long long* fa_ticket = nullptr;
+    // every member's strips fit the one-launch PCG (b_pcg_loop_kernel)
+    bool loop = false, any_loop = false;
+    unsigned long long* loop_ticket = nullptr;
     int* all_done_since = nullptr;
     const int* pcg_order = nullptr;  // members by SpMV/axpy virtual-workgroup weight, heaviest first (in d_maps)
     int* h_err = nullptr;
@@ -120,7 +123,7 @@ InstBufs inst_bufs(const fs2d_sim* s, unsigned long long* sk_handoff, unsigned* 
     I.cell = s->cell; I.cell2 = s->cell2; I.phi = s->phi; I.phi2 = s->phi2; I.t0 = s->t0; I.t1 = s->t1; I.ls_chg = s->ls_chg;
     I.p = s->p; I.r = s->r; I.z = s->z; I.q = s->q; I.w = s->w; I.s0 = s->s[0]; I.s1 = s->s[1]; I.pk = s->pk;
     I.Adiag = s->Adiag; I.P = s->P; I.fx = s->fx; I.fy = s->fy; I.G = s->G; I.cpl = s->cpl;
-    I.tile_act = s->tile_act; I.range = s->range; I.hrows = s->hrows;
+    I.tile_act = s->tile_act; I.range = s->range; I.hrows = s->hrows; I.loop_words = s->loop_words;
     I.sc = s->sc; I.qq = s->qq; I.ws_part = s->ws_part; I.rmax_part = s->rmax_part;
     I.mu = s->mu; I.mv = s->mv; I.fu0 = s->fu0; I.fu1 = s->fu1; I.fv0 = s->fv0; I.fv1 = s->fv1; I.fcount = s->fcount;
     I.fpos = s->fpos; I.fsrc = s->fsrc; I.fkv = s->fkv;
@@ -436,6 +439,7 @@ void bpcg_iterations(fs2d_batch* B, int h0, int h1, Fwd fwd, Bwd bwd) {
             hipLaunchKernelGGL(b_pcg_plan_kernel, dim3(B->n), dim3(kBlock), B->plan_lds, B->stream, B->d_ins, B->n,
                                B->m_pcg.count, B->pcg_order, B->plan, h, B->all_done_since);
             blaunch(B, b_spmv_kernel, B->pcg_grid, kBlock, B->d_ins, B->m_pcg.count, B->plan, h);
+            if (B->any_loop) blaunch(B, b_spmv_strip_kernel, S, kLoopThreads, B->d_ins, B->strips, h);
         }
         if (B->fused_pcg) {
             {
@@ -484,6 +488,13 @@ void bpcg_iterations(fs2d_batch* B, int h0, int h1) {
                         b_sweep_kernel<BwdOp, true, BwdMaker, true, false>);
 }
 
+// The PCG of every member in one launch (unless its kernels are timed): when
+// each member's strips fit it.
+bool bpcg_in_loop(const fs2d_batch* B) { return B->loop && !B->timing; }
+void bpcg_loop(fs2d_batch* B) {
+    blaunch(B, b_pcg_loop_kernel, B->strips.total, kLoopThreads, B->d_ins, B->strips, B->loop_ticket, B->werr);
+}
+
 // Assembly, MIC(0) factor and the first preconditioner application of every
 // member (FluidSim2D.cpp:252-430).
 void bpcg_begin(fs2d_batch* B) {
@@ -497,6 +508,10 @@ void bpcg_begin(fs2d_batch* B) {
         Timed t(B, K_FACTOR);
         blaunch(B, b_sweep_kernel<FactorOp, false, FactorMaker, true>, S, kSweepThreads, B->d_ins, B->strips,
                 B->sk_ticket, B->werr, FactorMaker{B->m_sk.count}, (const int*)nullptr, 0, (const int*)nullptr);
+    }
+    if (bpcg_in_loop(B)) {
+        bpcg_loop(B);
+        return;
     }
     {
         Timed t(B, K_PCG_FWD);
@@ -550,7 +565,7 @@ fs2d_status bpcg_status(fs2d_batch* B) {
 
 fs2d_status bstage_projection(fs2d_batch* B) {
     bpcg_begin(B);
-    TRY(bpcg_continue(B, 0, std::max(2, std::min(B->last_iters_hint, B->max_iters))));
+    if (!bpcg_in_loop(B)) TRY(bpcg_continue(B, 0, std::max(2, std::min(B->last_iters_hint, B->max_iters))));
     bpcg_end(B);
     TRY(gather_status(B));
     return bpcg_status(B);
@@ -675,7 +690,7 @@ fs2d_status bcapture_step(fs2d_batch* B, fs2d_batch::Captured& G) {
         if (st == FS2D_OK) st = bstage(B, stg, fuse, &worst);
     if (st == FS2D_OK) {
         bpcg_begin(B);
-        bpcg_iterations(B, 0, G.budget);
+        if (!bpcg_in_loop(B)) bpcg_iterations(B, 0, G.budget);
     }
     fs2d_status ce = bend_capture(B, &G.pre);
     if (st == FS2D_OK && ce == FS2D_OK) {
@@ -719,8 +734,8 @@ fs2d_status bstep_graph(fs2d_batch* B) {
         G = &B->graphs.back();
     }
     BHIPCHK(B, hipGraphLaunch(G->pre, B->stream));
-    TRY(gather_status(B));
-    if (!all_members_done(B) && G->budget < B->max_iters) TRY(bpcg_continue(B, G->budget, 8));
+    if (!bpcg_in_loop(B)) TRY(gather_status(B));
+    if (!bpcg_in_loop(B) && !all_members_done(B) && G->budget < B->max_iters) TRY(bpcg_continue(B, G->budget, 8));
     BHIPCHK(B, hipGraphLaunch(G->post, B->stream));
     TRY(gather_status(B));
     const fs2d_status pst = bpcg_status(B);
@@ -786,8 +801,11 @@ fs2d_status fs2d_batch_create(const fs2d_config* cfgs, int n, fs2d_batch** out) 
     // hand-off rows and descriptors, then the launch maps
     B->h_ins.resize(n);
     fs2d_status st = FS2D_OK;
+    B->loop = true;
     for (int b = 0; b < n; b++) {
         fs2d_sim* s = B->sims[b];
+        B->loop = B->loop && s->loop;
+        B->any_loop = B->any_loop || s->loop;
         const int ns = (s->ny + 63) / 64;
         unsigned long long* skh = nullptr;
         unsigned* faf = nullptr;
@@ -800,6 +818,7 @@ fs2d_status fs2d_batch_create(const fs2d_config* cfgs, int n, fs2d_batch** out) 
     if ((st = build_maps(B)) != FS2D_OK) return bail(st);
     if ((st = balloc(B, &B->werr, 1)) != FS2D_OK || (st = balloc(B, &B->all_done_since, 1)) != FS2D_OK ||
         (st = balloc(B, &B->sk_ticket, 1)) != FS2D_OK || (st = balloc(B, &B->fa_ticket, 1)) != FS2D_OK ||
+        (st = balloc(B, &B->loop_ticket, 1)) != FS2D_OK ||
         (st = balloc(B, &B->d_status, 4 * (size_t)n)) != FS2D_OK)
         return bail(st);
     B->plan_lds = sizeof(int) * (size_t)n;

@@ -109,6 +109,10 @@ struct fs2d_sim {
     // each launch cost 2% of a 1000 x 700 step and there is nothing to skip.
     bool use_range = true;
     HandRows hrows{};             // boundary rows of the solves
+    // The PCG as one launch (pcg_loop_kernel) where the grid's strips fit it;
+    // per-kernel timing takes its phases as separate launches.
+    bool loop = false;
+    unsigned long long* loop_words = nullptr;
     PcgScalars* sc = nullptr;
     PcgScalars* h_sc = nullptr;
     double *qq = nullptr, *ws_part = nullptr, *rmax_part = nullptr;
@@ -555,6 +559,11 @@ void assemble(fs2d_sim* s) {
                        1.0 / (s->dx * solver_scale(s)), s->rmax_part, ghost_pressure(s));
 }
 
+// Grids whose strips run the PCG in one launch (unless its kernels are timed:
+// then the launches below with its order of the sums), and those with two
+// launches per iteration.
+bool pcg_in_loop(const fs2d_sim* s) { return s->loop && !s->timing; }
+bool pcg_fused(const fs2d_sim* s) { return s->fused_pcg && !s->loop; }
 // Physical workgroups of the PCG SpMV and axpy launches: their loops run the
 // pcg_blocks virtual workgroups (pcg_grid 0: one each), so this choice
 // changes no result; a multiple of 8 (xcd_loop).
@@ -622,6 +631,7 @@ void pcg_begin(fs2d_sim* s) {
                     s->max_iters, s->sc, 1e-12 / solver_scale(s)};
         launch_sweep<FactorOp, false>(s, op, solve_range(s));
     }
+    if (pcg_in_loop(s)) return;
     {
         Timed t(s, K_PCG_FWD);
         FwdOp op{{s->r, s->P, s->fx, s->fy}, nullptr, {s->q}, s->hrows.set(s->geom, false, 0),
@@ -630,7 +640,7 @@ void pcg_begin(fs2d_sim* s) {
     }
     {
         Timed t(s, K_PCG_BWD);
-        if (s->fused_pcg) {
+        if (pcg_fused(s)) {
             launch_bwd_spmv(s, 0, s->qq, nullptr, 1, s->s[0], s->s[1], 0);
         } else {
             BwdOp op{{s->q, s->P, s->G}, nullptr, {s->z}, s->hrows.set(s->geom, true, 0),
@@ -657,7 +667,7 @@ void pcg_iterations(fs2d_sim* s, int h0, int h1) {
         float* s_new = s->s[(h + 1) & 1];
         double* sig_cur = (h & 1) ? qq1 : qq0;   // sigma_h
         double* sig_prev = (h & 1) ? qq0 : qq1;  // sigma_{h-1}; receives sigma_{h+1}
-        if (s->fused_pcg) {
+        if (pcg_fused(s)) {
             {
                 Timed t(s, K_PCG_FWD);
                 launch_fwd_axpy(s, h, s_new, sig_cur);
@@ -668,14 +678,19 @@ void pcg_iterations(fs2d_sim* s, int h0, int h1) {
         }
         {
             Timed t(s, K_PCG_SPMV);
-            hipLaunchKernelGGL(pcg_spmv_sk_kernel, dim3(grid), dim3(kBlock), 0, s->stream, g, s->Adiag, s->cpl, s->z,
+            if (s->loop)
+                hipLaunchKernelGGL(pcg_spmv_strip_kernel, dim3(g.S), dim3(kLoopThreads), 0, s->stream, g, s->Adiag,
+                                   s->z, s_old, s_new, s->w, s->sc, sig_cur, sig_prev, h == 0 ? 1 : 0,
+                                   s->ws_part, (const int2*)s->range);
+            else
+                hipLaunchKernelGGL(pcg_spmv_sk_kernel, dim3(grid), dim3(kBlock), 0, s->stream, g, s->Adiag, s->cpl, s->z,
                                s_old, s_new, s->w, s->sc, sig_cur, sig_prev, h == 0 ? 1 : 0, s->ws_part,
                                nbp);
         }
         {
             Timed t(s, K_PCG_AXPY);
             hipLaunchKernelGGL(pcg_axpy_sk_kernel, dim3(grid), dim3(kBlock), 0, s->stream, g, s->pk, s->r, s_new,
-                               s->w, s->sc, sig_cur, s->ws_part, nbp, s->rmax_part, nbp);
+                               s->w, s->sc, sig_cur, s->ws_part, s->loop ? g.S : nbp, s->rmax_part, nbp);
         }
         {
             Timed t(s, K_PCG_FWD);
@@ -699,11 +714,19 @@ void pcg_end(fs2d_sim* s, float* out) {
                        out);
 }
 
-// The whole PCG: the host reads the stopping flag once per chunk of queued
-// iterations (the first chunk sized by the previous solve's count).
+void launch_pcg_loop(fs2d_sim* s) {
+    const LoopArgs A{s->geom, s->Adiag, s->r,  s->pk,          s->s[0],  s->s[1],       s->w,        s->z, s->q, s->P,
+                     s->fx,   s->fy,    s->G,   s->sc, s->range,       s->hrows, s->loop_words, s->max_iters};
+    hipLaunchKernelGGL(pcg_loop_kernel, dim3(s->geom.S), dim3(kLoopThreads), 0, s->stream, A, s->werr);
+}
+
+// The whole PCG: one launch, or, where it does not fit, chunks of queued
+// iterations with one host read of the stopping flag each (the first chunk
+// sized by the previous solve's count).
 fs2d_status pcg_solve(fs2d_sim* s, float* out) {
     pcg_begin(s);
-    int h = 0;
+    if (pcg_in_loop(s)) launch_pcg_loop(s);
+    int h = pcg_in_loop(s) ? s->max_iters : 0;
     int batch = std::max(2, std::min(s->last_iters_hint, s->max_iters));
     while (h < s->max_iters) {
         const int nbatch = std::min(batch, s->max_iters - h);
@@ -874,7 +897,8 @@ fs2d_status capture_step(fs2d_sim* s, StepGraph& G) {
     if (st == FS2D_OK) {
         assemble(s);
         pcg_begin(s);
-        pcg_iterations(s, 0, G.budget);
+        if (pcg_in_loop(s)) launch_pcg_loop(s);
+        else pcg_iterations(s, 0, G.budget);
     }
     fs2d_status ce = end_capture(s, &G.pre);
     if (st == FS2D_OK && ce == FS2D_OK) {
@@ -923,7 +947,16 @@ fs2d_status step_graph(fs2d_sim* s) {
         G = &s->graphs.back();
     }
     HIPCHK(s, hipGraphLaunch(G->pre, s->stream));
-    TRY(d2h(s, s->h_sc, s->sc, sizeof(PcgScalars)));
+    if (pcg_in_loop(s)) {
+        // the solve ends inside `pre`: no host check between the graphs
+        HIPCHK(s, hipGraphLaunch(G->post, s->stream));
+        graph_restore(s, G->after);
+        TRY(d2h(s, s->h_sc, s->sc, sizeof(PcgScalars)));
+        s->last_iters_hint = std::max(2, s->h_sc->iter + 1);
+        s->current_time += s->dt;
+        s->steps++;
+        return finish(s, s->h_sc->iter >= s->max_iters ? FS2D_WARN_MAXITER : FS2D_OK);
+    }
     int h = G->budget;
     while (!s->h_sc->done && h < s->max_iters) {
         const int n = std::min(8, s->max_iters - h);
@@ -1110,6 +1143,8 @@ fs2d_status fs2d_create(const fs2d_config* cfg, fs2d_sim** out) {
     A(fa_ticket, 1); A(fa_flags, kMaxBlocks);
 #undef A
     if (hipDeviceGetAttribute(&s->ncu, hipDeviceAttributeMultiprocessorCount, s->device) != hipSuccess) s->ncu = 0;
+    s->loop = loop_fits(s->geom, s->ncu);
+    if (s->loop && (st = dalloc(s, &s->loop_words, loop_words(s->geom))) != FS2D_OK) return bail(st);
     e = hipHostMalloc((void**)&s->h_sc, sizeof(PcgScalars), hipHostMallocDefault);
     if (e == hipSuccess) e = hipHostMalloc((void**)&s->h_dg, sizeof(Diag), hipHostMallocDefault);
     if (e == hipSuccess) e = hipHostMalloc((void**)&s->h_err, sizeof(int), hipHostMallocDefault);
@@ -1621,10 +1656,12 @@ constexpr size_t kNaPart = na_align(sizeof(double) * kMaxBlocks);
 constexpr size_t kNaWord = 256;
 constexpr size_t kNaTiles = na_align(kNoallocEntries / 2048);
 constexpr size_t kNaRows = na_align(sizeof(uint32_t) * 4 * (kNoallocEntries / 64));
+// strips of at most kLoopMaxStrips and 4 T4 <= kLoopSteps
+constexpr size_t kNaLoop = na_align(sizeof(unsigned long long) * kLoopMaxStrips * (kLoopWords + kLoopSteps));
 constexpr size_t kNaRange = na_align(sizeof(int2) * kNoallocMaxStrips);
 constexpr size_t kNaHand = na_align(sizeof(unsigned long long) * kNoallocHandWords);
 constexpr size_t kNoallocBytes =
-    kNoallocFloatArrays * kNaFloats + kNaCpl + kNaSc + kNaQq + 2 * kNaPart + 2 * kNaWord + kNaTiles + kNaRange + kNaRows + kNaHand;
+    kNoallocFloatArrays * kNaFloats + kNaCpl + kNaSc + kNaQq + 2 * kNaPart + 2 * kNaWord + kNaTiles + kNaRange + kNaRows + kNaLoop + kNaHand;
 
 __device__ __align__(256) unsigned char scratch[kNoallocBytes];
 
@@ -1722,6 +1759,9 @@ fs2d_status fs2d_project_noalloc(const fs2d_projection_args* a, int* iters, doub
     t.tile_act = q;                              q += kNaTiles;
     t.range = (int2*)q;                          q += kNaRange;
     t.hrows.base = (uint32_t*)q;                 q += kNaRows;
+    t.loop_words = (unsigned long long*)q;       q += kNaLoop;
+    if (hipDeviceGetAttribute(&t.ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) t.ncu = 0;
+    t.loop = loop_fits(geom, t.ncu);
     t.sk_handoff = (unsigned long long*)q;
     t.fused_pcg = false;  // the separate SpMV launch: no completion flags or tagged sigma in the scratch
     PcgScalars h_sc{};

@@ -16,7 +16,8 @@ constexpr int kSpinLimit = 1 << 16;  // polls of one memory round trip each: wel
 // Bounded waits that expire raise the error flag; the first one's site stays in
 // it, so the host's message can name what was waited for.
 enum WaitSite {
-    kWaitCompute = 1, kWaitLoader, kWaitPollerRing, kWaitHandoff, kWaitRuns, kWaitSigma, kWaitStrip, kWaitStrips
+    kWaitCompute = 1, kWaitLoader, kWaitPollerRing, kWaitHandoff, kWaitRuns, kWaitSigma, kWaitStrip, kWaitStrips,
+    kWaitArrive, kWaitLoopWords, kWaitLoopRow
 };
 __device__ __forceinline__ void raise_wait(int* err, int site) { atomicCAS(err, 0, site); }
 

@@ -1116,6 +1116,7 @@ __global__ __launch_bounds__(64) void pcg_init_kernel(PcgScalars* sc, double tol
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         PcgScalars z{};
         z.tol = tol;
+        z.epoch = sc->epoch + (unsigned)sc->iter + 4u;  // past every tag of the previous solve
         *sc = z;
     }
 }

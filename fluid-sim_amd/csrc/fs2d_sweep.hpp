@@ -513,13 +513,20 @@ __device__ __forceinline__ unsigned long long sweep_ticket(SweepLds<Op, RING>& L
 // One strip of a pass: `order` is the strip's position in the pass (strip
 // order for forward passes, reversed for backward ones), `epoch` tags its
 // hand-off words.
-template <class Op, bool BACKWARD, bool PREFETCH, int RING>
+// LOOP: one pass of many by a workgroup that keeps its strip (`order` is the
+// strip, fs2d_pcg_loop.hpp): no stopping test, the LDS counters are set here,
+// and the wave past the pollers calls spare() meanwhile.  The caller has a
+// barrier before and after.
+struct NoSpare {
+    __device__ void operator()() const {}
+};
+template <class Op, bool BACKWARD, bool PREFETCH, int RING, bool LOOP = false, class Spare = NoSpare>
 __device__ __forceinline__ void sweep_run(Op& op, const SkGeom& g, const SkCtl& c, int order, unsigned epoch,
-                                          SweepLds<Op, RING>& L) {
+                                          SweepLds<Op, RING>& L, Spare spare = Spare{}) {
     constexpr int NW = Op::NW, NIN = Op::NIN, NF = Op::NF, NB = Op::NB;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     __shared__ int sh_skip;
-    const int s = BACKWARD ? g.S - 1 - order : order;
+    const int s = BACKWARD && !LOOP ? g.S - 1 - order : order;
     const StripSpan sp = strip_span<BACKWARD>(g, c.range, s);
     const int T = g.T4 * 4, nx = g.nx;
 
@@ -550,7 +557,13 @@ __device__ __forceinline__ void sweep_run(Op& op, const SkGeom& g, const SkCtl& 
         if constexpr (waits_inputs<Op>()) op.wait_inputs(s, c.err);
         if (PREFETCH) load_sg(sg0);
     }
-    if (wave == 0) {
+    if (LOOP) {
+        if (threadIdx.x == 0) {
+            L.consumed_sg = (unsigned)sp.lo;
+            L.hand_ready = 0;
+        }
+        if (threadIdx.x < RING) L.slot_tag[threadIdx.x] = 0;
+    } else if (wave == 0) {
         int sk = __hip_atomic_load(c.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
         if (!sk) sk = op.skip(order == 0);
         if (lane == 0) {
@@ -559,7 +572,7 @@ __device__ __forceinline__ void sweep_run(Op& op, const SkGeom& g, const SkCtl& 
         }
     }
     __syncthreads();
-    if (sh_skip) return;
+    if (!LOOP && sh_skip) return;
     if (sp.lo >= sp.hi) {  // nothing in this strip
         if (wave == 0) op.strip_done(s);
         else if (wave <= kLoaders) op.loader_done(s, me, 0.0);
@@ -626,6 +639,8 @@ __device__ __forceinline__ void sweep_run(Op& op, const SkGeom& g, const SkCtl& 
             if (lane == 0) lds_st(&L.slot_tag[slot], (unsigned)sg + 1u);
         }
         op.loader_done(s, me, acc);
+    } else if (wave > kLoaders + kPollers) {
+        spare();
     } else if (sp.consume) {
         // ------------------------------------------------------------- pollers
         // Steps in consumption order kk = 16 lo .. 16 hi - 1 (step t = kk
@@ -697,6 +712,11 @@ __device__ __forceinline__ void sweep_run(Op& op, const SkGeom& g, const SkCtl& 
             }
         }
     }
+    if (LOOP) {  // rows reset, results stored
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(kWaitVm0);
+        asm volatile("" ::: "memory");
+    }
 }
 
 // Supergroups in a single launch's ring: kRing, or 4 for operators with more
@@ -729,7 +749,7 @@ struct PcgScalars {
     int done;  // 0: iterating.  Non-zero: stopped; the launch whose stopping test runs beside
                // strips that read this (bwd_spmv_kernel) writes its next_iter + 1 (>= 2)
     float beta;  // beta of the current iteration when a separate reduction formed it
-    int pad1;
+    unsigned epoch;  // tags of a solve in one launch: epoch + iteration (fs2d_pcg_loop.hpp)
 };
 
 __device__ __forceinline__ double wave_max_of(const double* a, int n) {
