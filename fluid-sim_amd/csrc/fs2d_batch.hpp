@@ -669,7 +669,8 @@ __global__ __launch_bounds__(kSweepThreads) void b_sweep_kernel(const InstBufs* 
 // waits only for its own simulation, and a workgroup that finishes makes room
 // for the next member's.  Strips are taken in the order of the strip list.
 __global__ __launch_bounds__(kLoopThreads) void b_pcg_loop_kernel(const InstBufs* __restrict__ ins, StripMap sm,
-                                                                  unsigned long long* ticket, int* err) {
+                                                                  int max_iters, unsigned long long* ticket,
+                                                                  int* err) {
     __shared__ __align__(16) LoopLds L;
     __shared__ unsigned long long sh_ticket;
     if (threadIdx.x == 0) sh_ticket = atomicAdd(ticket, 1ull);
@@ -677,8 +678,8 @@ __global__ __launch_bounds__(kLoopThreads) void b_pcg_loop_kernel(const InstBufs
     const int gs = (int)uniform((unsigned)(sh_ticket % (unsigned long long)sm.total));
     const int b = sm.inst[gs];
     const InstBufs& I = ins[b];
-    const LoopArgs A{I.geom, I.Adiag, I.r, I.pk, I.s0,    I.s1,    I.w,          I.z,        I.q, I.P,
-                     I.fx,   I.fy,    I.G,   I.sc, I.range, I.hrows, I.loop_words, I.max_iters};
+    const LoopArgs A{I.geom, I.Adiag, I.r, I.pk, I.s0,    I.s1,    I.w,          I.z,      I.q, I.P,
+                     I.fx,   I.fy,    I.G, I.sc, I.range, I.hrows, I.loop_words, max_iters};
     pcg_loop_strip(A, gs - sm.first[b], L, err);
 }
 

@@ -492,7 +492,8 @@ void bpcg_iterations(fs2d_batch* B, int h0, int h1) {
 // each member's strips fit it.
 bool bpcg_in_loop(const fs2d_batch* B) { return B->loop && !B->timing; }
 void bpcg_loop(fs2d_batch* B) {
-    blaunch(B, b_pcg_loop_kernel, B->strips.total, kLoopThreads, B->d_ins, B->strips, B->loop_ticket, B->werr);
+    blaunch(B, b_pcg_loop_kernel, B->strips.total, kLoopThreads, B->d_ins, B->strips, B->max_iters, B->loop_ticket,
+            B->werr);
 }
 
 // Assembly, MIC(0) factor and the first preconditioner application of every

@@ -26,14 +26,17 @@
 //   waves 1..L      loaders: stream the strip's inputs (SK4 layout, 1 KB per
 //                   wave-wide dwordx4 load), apply the operator's per-cell
 //                   transform (e.g. P*r) and fill an LDS ring of supergroups.
-//   wave L+1        poller: reads the neighbouring strip's boundary row from
-//                   tagged 64-bit words ({payload, epoch}, agent-scope relaxed
-//                   atomics, see fs2d_gmem.hpp) into an LDS ring indexed
-//                   by step; steps whose edge column is outside the grid get
-//                   the boundary value.
-// The producing lane's 16 boundary values per supergroup go through a 2-entry
-// LDS outbox and are stored as tagged words by 16 lanes after the first
-// sub-group of the next supergroup, into a padded row (no range tests).
+//   waves L+1, L+2  pollers: read the neighbouring strip's boundary row into an
+//                   LDS ring indexed by step: the solves' from untagged words
+//                   that hold kUnset until written (HandRows), the other
+//                   passes' from tagged words ({payload, epoch}), both with
+//                   agent-scope relaxed atomics (fs2d_gmem.hpp); steps whose
+//                   edge column is outside the grid get the boundary value.
+// The solves' producing lane stores its row with the buffer stores of the step
+// (other lanes' offsets are out of range).  In the other passes its 16 boundary
+// values per supergroup go through a 2-entry LDS outbox and are stored as
+// tagged words by 16 lanes after the first sub-group of the next supergroup,
+// into a padded row (no range tests).
 //
 // Waves signal each other through LDS counters without s_waitcnt: LDS executes
 // one wave's operations in order, so a flag written after data (or after the
