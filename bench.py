@@ -102,17 +102,17 @@ PROFILE_STEPS = 2  # steps with every kernel class timed, outside the timed regi
 # hits by design).  FP32 fields, uint8 flags, FP64 level set.
 BYTES_PER_CELL = {
     "pcg_forward_solve": 20,    # r, P, fx, fy in; q out
-    "pcg_backward_solve": 20,   # q, P, gx, gy in; z out
-    # the backward solve with the next SpMV in one launch: q, P, gx, gy in, z
+    "pcg_backward_solve": 16,   # q, P, G in; z out
+    # the backward solve with the next SpMV in one launch: q, P, G in, z
     # out; s, Adiag, coupling byte in, s', w out (z and q counted once)
-    "pcg_backward_solve+spmv": 37,
+    "pcg_backward_solve+spmv": 33,
     # the p/r update with the forward solve in one launch: p, r, s, w in, p, r
     # out; P, fx, fy in, q out (r counted once each way)
     "pcg_forward_solve+axpy": 40,
     "pcg_spmv_dot": 21,         # z, s, Adiag, coupling byte in; s', w out
     "pcg_axpy_norm": 24,        # p, r, s, w in; p, r out
-    "mic0_factor": 25,          # Adiag, coupling byte in; P, fx, fy, gx, gy out
-    "assemble": 34,             # cell, phi (f64), u, v in; Adiag, coupling, r, p, s out
+    "mic0_factor": 21,          # Adiag, coupling byte in; P, fx, fy, G out
+    "assemble": 38,             # cell, phi (f64), u, v in; Adiag, coupling, r, p, s, z out
     "sl_advect": 24,            # u, v, density in and out
 }
 # launches that did work per step: `iters` loop launches (+1 initial solve)

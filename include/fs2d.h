@@ -242,6 +242,9 @@ const char* fs2d_status_string(int status);
  *     The loops run a fixed list of virtual workgroups whatever the launch
  *     size, so every value gives the same bits.  Unused by fused_pcg
  *     iterations, whose launches size themselves to the device.
+ *     Grids of at most 1024 rows and 576 columns, and ensembles of them, run
+ *     the whole PCG in one launch, which uses neither pcg_grid nor fused_pcg
+ *     (unless per-kernel timing is on).
  *   sweep_prefetch: (ensembles) the batched triangular solves' loaders issue
  *     their first loads before testing whether their member has converged.
  *   fused_pcg: (single handles) 1, the default for solver layouts of at least
@@ -278,7 +281,8 @@ fs2d_status fs2d_autotune(fs2d_sim* sim, int iters, const char* cache_path, fs2d
  * tight serving loops, harnesses that forbid hipMalloc).  It runs the
  * ghost-fluid assembly, the MIC(0) factor and the PCG of
  * fs2d_run_stage(sim, FS2D_STAGE_APPLY_PROJECTION) (src/FluidSim2D.cpp:252-467),
- * with four launches per PCG iteration (fused_pcg 0, whatever the grid), on the
+ * with the whole PCG in one launch where the grid fits it (see fs2d_tuning) and
+ * four launches per iteration elsewhere (fused_pcg 0), on the
  * caller's device arrays and gives the same pressure bit for bit.  Every other array
  * lives in a static device buffer of about 28 MB per GPU, held from the
  * library's load until the process ends; grids whose solver layout has at most
