@@ -336,6 +336,10 @@ __device__ __forceinline__ void pcg_loop_strip(const LoopArgs& A, int s, LoopLds
     const int2 rd = below ? L.range[s - 1] : make_int2(0, 0), ru = above ? L.range[s + 1] : make_int2(0, 0);
     double sig_prev = 0, rn = A.sc->rhs_norm;
     int iter = 0, done = 0;
+    // after an expired wait: the next solve's tags start past those in use here
+    auto fail = [&](int it) {
+        if (tid == 0) atomicMax(&A.sc->iter, it);
+    };
     for (int it = 0;; it++) {
         const unsigned tag = tag0 + (unsigned)it;
         const unsigned long long tagw = (unsigned long long)tag << 32;
@@ -366,7 +370,7 @@ __device__ __forceinline__ void pcg_loop_strip(const LoopArgs& A, int s, LoopLds
             });
         }
         __syncthreads();
-        if (L.bad || L.fwd.abort_flag) return;
+        if (L.bad || L.fwd.abort_flag) return fail(it);
         if (it > 0) {
             rn = L.rn;
             if (rn <= stop) {
@@ -390,7 +394,7 @@ __device__ __forceinline__ void pcg_loop_strip(const LoopArgs& A, int s, LoopLds
             sweep_run<LoopBwdOp, true, true, kRing, true>(op, g, ctl, s, 0, L.bwd);
         }
         __syncthreads();
-        if (L.bwd.abort_flag) return;
+        if (L.bwd.abort_flag) return fail(it);
         iter = it;
         if (it >= A.max_iters) break;
 
@@ -440,7 +444,7 @@ __device__ __forceinline__ void pcg_loop_strip(const LoopArgs& A, int s, LoopLds
             }
         }
         __syncthreads();
-        if (L.bad) return;
+        if (L.bad) return fail(it);
         const double sig = L.sig;
         const float beta = it > 0 ? (float)(sig / sig_prev) : 0.0f;
         sig_prev = sig;
@@ -468,7 +472,7 @@ __device__ __forceinline__ void pcg_loop_strip(const LoopArgs& A, int s, LoopLds
             if (lane == 0) L.ws = ws;
         }
         __syncthreads();
-        if (L.bad) return;
+        if (L.bad) return fail(it);
         // alpha = sigma / w.s' (:450); p += alpha s', r -= alpha w (:451-452)
         const float alpha = (float)(sig / L.ws);
         float m = 0.0f;
