@@ -957,6 +957,7 @@ fs2d_status step_graph(fs2d_sim* s) {
         s->steps++;
         return finish(s, s->h_sc->iter >= s->max_iters ? FS2D_WARN_MAXITER : FS2D_OK);
     }
+    TRY(d2h(s, s->h_sc, s->sc, sizeof(PcgScalars)));
     int h = G->budget;
     while (!s->h_sc->done && h < s->max_iters) {
         const int n = std::min(8, s->max_iters - h);
