@@ -488,10 +488,10 @@ void bpcg_iterations(fs2d_batch* B, int h0, int h1) {
                         b_sweep_kernel<BwdOp, true, BwdMaker, true, false>);
 }
 
-// The PCG of every member in one launch (unless its kernels are timed): when
-// each member's strips fit it.
-bool bpcg_in_loop(const fs2d_batch* B) { return B->loop && !B->timing; }
+// The PCG of every member in one launch: when each member's strips fit it.
+bool bpcg_in_loop(const fs2d_batch* B) { return B->loop; }
 void bpcg_loop(fs2d_batch* B) {
+    Timed t(B, K_PCG_LOOP);
     blaunch(B, b_pcg_loop_kernel, B->strips.total, kLoopThreads, B->d_ins, B->strips, B->max_iters, B->loop_ticket,
             B->werr);
 }

@@ -29,13 +29,15 @@ namespace {
 enum KernelClass {
     K_SL_ADVECT, K_GRAVITY, K_ASSEMBLE, K_FACTOR, K_PCG_FWD, K_PCG_BWD, K_PCG_SPMV, K_PCG_AXPY,
     K_UPDATE_VEL, K_EXTRAPOLATE, K_PARTICLE_SORT, K_P2G, K_G2P, K_PARTICLE_ADVECT,
-    K_LS_SWEEP, K_LS_OTHER, K_DIAGNOSTICS, K_MISC, K_ADJ_SL, K_ADJ_OTHER, K_COUNT
+    K_LS_SWEEP, K_LS_OTHER, K_DIAGNOSTICS, K_MISC, K_ADJ_SL, K_ADJ_OTHER, K_PCG_LOOP, K_COUNT
 };
+// Classes of the PCG by launches per iteration.
+constexpr unsigned long long kPcgPhases = 1ull << K_PCG_FWD | 1ull << K_PCG_BWD | 1ull << K_PCG_SPMV | 1ull << K_PCG_AXPY;
 const char* kKernelNames[K_COUNT] = {
     "sl_advect", "gravity", "assemble", "mic0_factor", "pcg_forward_solve", "pcg_backward_solve",
     "pcg_spmv_dot", "pcg_axpy_norm", "update_velocity", "extrapolate", "particle_sort", "p2g", "g2p",
     "particle_advect", "levelset_sweep", "levelset_other", "diagnostics", "misc", "adjoint_sl",
-    "adjoint_other"};
+    "adjoint_other", "pcg_one_launch"};
 
 constexpr int kMaxBlocks = 2048;
 // Solver layouts of at least this many entries (a 512^2 grid has 294912) run
@@ -110,7 +112,7 @@ struct fs2d_sim {
     bool use_range = true;
     HandRows hrows{};             // boundary rows of the solves
     // The PCG as one launch (pcg_loop_kernel) where the grid's strips fit it;
-    // per-kernel timing takes its phases as separate launches.
+    // timing any of kPcgPhases takes its phases as separate launches.
     bool loop = false;
     unsigned long long* loop_words = nullptr;
     PcgScalars* sc = nullptr;
@@ -559,10 +561,10 @@ void assemble(fs2d_sim* s) {
                        1.0 / (s->dx * solver_scale(s)), s->rmax_part, ghost_pressure(s));
 }
 
-// Grids whose strips run the PCG in one launch (unless its kernels are timed:
+// Grids whose strips run the PCG in one launch (unless its phases are timed:
 // then the launches below with its order of the sums), and those with two
 // launches per iteration.
-bool pcg_in_loop(const fs2d_sim* s) { return s->loop && !s->timing; }
+bool pcg_in_loop(const fs2d_sim* s) { return s->loop && !(s->timing & kPcgPhases); }
 bool pcg_fused(const fs2d_sim* s) { return s->fused_pcg && !s->loop; }
 // Physical workgroups of the PCG SpMV and axpy launches: their loops run the
 // pcg_blocks virtual workgroups (pcg_grid 0: one each), so this choice
@@ -715,6 +717,7 @@ void pcg_end(fs2d_sim* s, float* out) {
 }
 
 void launch_pcg_loop(fs2d_sim* s) {
+    Timed t(s, K_PCG_LOOP);
     const LoopArgs A{s->geom, s->Adiag, s->r,  s->pk,          s->s[0],  s->s[1],       s->w,        s->z, s->q, s->P,
                      s->fx,   s->fy,    s->G,   s->sc, s->range,       s->hrows, s->loop_words, s->max_iters};
     hipLaunchKernelGGL(pcg_loop_kernel, dim3(s->geom.S), dim3(kLoopThreads), 0, s->stream, A, s->werr);

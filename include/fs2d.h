@@ -218,12 +218,17 @@ fs2d_status fs2d_set_graph(fs2d_sim* sim, int enable);
 
 /* Per-kernel timing with HIP events on the handle's stream (no reference
  * counterpart; PerformanceCounter, src/PerformanceCounter.cpp:9-74, timed
- * stages with a host clock).  Kernel classes are listed by fs2d_kernel_name. */
+ * stages with a host clock).  Kernel classes are listed by fs2d_kernel_name.
+ * A PCG that runs in one launch (see fs2d_tuning) is class pcg_one_launch.
+ * Timing any of pcg_forward_solve, pcg_backward_solve, pcg_spmv_dot and
+ * pcg_axpy_norm, as fs2d_set_timing(sim, 1) does, runs it by launches per
+ * iteration instead: the same bits, in more time. */
 fs2d_status fs2d_set_timing(fs2d_sim* sim, int enable);
 /* Times only the kernel classes whose bit is set in class_mask (bit k: class k
  * of fs2d_kernel_name; 0 turns timing off).  Each timed launch records two
  * events on the stream, which costs the step time: timing one class measures
- * that class while leaving the others untouched.  No reference counterpart. */
+ * that class while leaving the others untouched (the four PCG classes above
+ * excepted).  No reference counterpart. */
 fs2d_status fs2d_set_timing_classes(fs2d_sim* sim, unsigned long long class_mask);
 int fs2d_kernel_count(void);
 const char* fs2d_kernel_name(int kernel);
@@ -244,7 +249,7 @@ const char* fs2d_status_string(int status);
  *     iterations, whose launches size themselves to the device.
  *     Grids of at most 1024 rows and 576 columns, and ensembles of them, run
  *     the whole PCG in one launch, which uses neither pcg_grid nor fused_pcg
- *     (unless per-kernel timing is on).
+ *     (unless one of its phases is timed, fs2d_set_timing).
  *   sweep_prefetch: (ensembles) the batched triangular solves' loaders issue
  *     their first loads before testing whether their member has converged.
  *   fused_pcg: (single handles) 1, the default for solver layouts of at least
@@ -382,7 +387,8 @@ fs2d_status fs2d_batch_get_tuning(fs2d_batch* batch, fs2d_tuning* out);
 fs2d_status fs2d_batch_set_tuning(fs2d_batch* batch, const fs2d_tuning* t);
 fs2d_status fs2d_batch_autotune(fs2d_batch* batch, int iters, const char* cache_path, fs2d_tuning* out,
                                 int* from_cache);
-/* Per-kernel timing of the batched launches (kernel classes of fs2d_kernel_name). */
+/* Per-kernel timing of the batched launches (kernel classes of fs2d_kernel_name):
+ * of those that untimed steps run, the PCG in one launch included. */
 fs2d_status fs2d_batch_set_timing(fs2d_batch* batch, int enable);
 fs2d_status fs2d_batch_get_kernel_time(fs2d_batch* batch, int kernel, double* total_ms, long long* launches);
 fs2d_status fs2d_batch_reset_kernel_times(fs2d_batch* batch);
