@@ -48,6 +48,7 @@ struct fs2d_batch {
     unsigned long long* fa_ticket = nullptr;
     // every member's strips fit the one-launch PCG (b_pcg_loop_kernel)
     bool loop = false, any_loop = false;
+    bool room = true;  // loop_room of the batch's stream
     unsigned long long* loop_ticket = nullptr;
     int* all_done_since = nullptr;
     const int* pcg_order = nullptr;  // members by SpMV/axpy virtual-workgroup weight, heaviest first (in d_maps)
@@ -488,8 +489,9 @@ void bpcg_iterations(fs2d_batch* B, int h0, int h1) {
                         b_sweep_kernel<BwdOp, true, BwdMaker, true, false>);
 }
 
-// The PCG of every member in one launch: when each member's strips fit it.
-bool bpcg_in_loop(const fs2d_batch* B) { return B->loop; }
+// The PCG of every member in one launch: when each member's strips fit it, and
+// there is room for it.
+bool bpcg_in_loop(const fs2d_batch* B) { return B->loop && B->room; }
 void bpcg_loop(fs2d_batch* B) {
     Timed t(B, K_PCG_LOOP);
     blaunch(B, b_pcg_loop_kernel, B->strips.total, kLoopThreads, B->d_ins, B->strips, B->max_iters, B->loop_ticket,
@@ -803,6 +805,7 @@ fs2d_status fs2d_batch_create(const fs2d_config* cfgs, int n, fs2d_batch** out) 
     B->h_ins.resize(n);
     fs2d_status st = FS2D_OK;
     B->loop = true;
+    B->room = stream_room(B->stream, B->sims[0]->ncu);
     for (int b = 0; b < n; b++) {
         fs2d_sim* s = B->sims[b];
         B->loop = B->loop && s->loop;

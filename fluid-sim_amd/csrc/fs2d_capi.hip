@@ -114,6 +114,7 @@ struct fs2d_sim {
     // The PCG as one launch (pcg_loop_kernel) where the grid's strips fit it;
     // timing any of kPcgPhases takes its phases as separate launches.
     bool loop = false;
+    bool room = true;  // loop_room of the handle's stream
     unsigned long long* loop_words = nullptr;
     PcgScalars* sc = nullptr;
     PcgScalars* h_sc = nullptr;
@@ -561,10 +562,24 @@ void assemble(fs2d_sim* s) {
                        1.0 / (s->dx * solver_scale(s)), s->rmax_part, ghost_pressure(s));
 }
 
-// Grids whose strips run the PCG in one launch (unless its phases are timed:
-// then the launches below with its order of the sums), and those with two
-// launches per iteration.
-bool pcg_in_loop(const fs2d_sim* s) { return s->loop && !(s->timing & kPcgPhases); }
+// loop_room of a stream, with the CUs that its mask (its own, or the process's)
+// leaves it, and HIP's hardware queues: 4, unless the environment asks for others.
+bool stream_room(hipStream_t stream, int ncu) {
+    uint32_t mask[64] = {};
+    int cus = 0;
+    if (hipExtStreamGetCUMask(stream, 64, mask) == hipSuccess)
+        for (uint32_t m : mask) cus += __builtin_popcount(m);
+    else
+        (void)hipGetLastError();
+    if (cus == 0) cus = ncu;
+    const char* e = getenv("GPU_MAX_HW_QUEUES");
+    const int queues = e ? std::clamp(atoi(e), 0, 4096) : 0;
+    return loop_room(std::min(cus, ncu), queues > 0 ? queues : 4);
+}
+// Grids whose strips run the PCG in one launch (unless its phases are timed, or
+// there is no room for it: then the launches below with its order of the sums),
+// and those with two launches per iteration.
+bool pcg_in_loop(const fs2d_sim* s) { return s->loop && s->room && !(s->timing & kPcgPhases); }
 bool pcg_fused(const fs2d_sim* s) { return s->fused_pcg && !s->loop; }
 // Physical workgroups of the PCG SpMV and axpy launches: their loops run the
 // pcg_blocks virtual workgroups (pcg_grid 0: one each), so this choice
@@ -1148,6 +1163,7 @@ fs2d_status fs2d_create(const fs2d_config* cfg, fs2d_sim** out) {
 #undef A
     if (hipDeviceGetAttribute(&s->ncu, hipDeviceAttributeMultiprocessorCount, s->device) != hipSuccess) s->ncu = 0;
     s->loop = loop_fits(s->geom, s->ncu);
+    s->room = stream_room(s->stream, s->ncu);
     if (s->loop && (st = dalloc(s, &s->loop_words, loop_words(s->geom))) != FS2D_OK) return bail(st);
     e = hipHostMalloc((void**)&s->h_sc, sizeof(PcgScalars), hipHostMallocDefault);
     if (e == hipSuccess) e = hipHostMalloc((void**)&s->h_dg, sizeof(Diag), hipHostMallocDefault);
@@ -1766,6 +1782,7 @@ fs2d_status fs2d_project_noalloc(const fs2d_projection_args* a, int* iters, doub
     t.loop_words = (unsigned long long*)q;       q += kNaLoop;
     if (hipDeviceGetAttribute(&t.ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) t.ncu = 0;
     t.loop = loop_fits(geom, t.ncu);
+    t.room = stream_room(t.stream, t.ncu);
     t.sk_handoff = (unsigned long long*)q;
     t.fused_pcg = false;  // the separate SpMV launch: no completion flags or tagged sigma in the scratch
     PcgScalars h_sc{};

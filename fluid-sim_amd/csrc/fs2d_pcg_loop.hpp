@@ -28,7 +28,8 @@
 // kLoopMaxStrips workgroups while it waits for earlier simulations (which
 // finish without it) or other streams' kernels to leave.  With one workgroup
 // per CU, 256 CUs and HIP's 4 hardware queues, 16 strips leave room four times
-// over; a device with fewer CUs takes the separate launches (loop_fits).
+// over; a device with fewer CUs takes the separate launches (loop_fits), and so
+// do a process that asks for more queues and a stream with few CUs (loop_room).
 #pragma once
 
 #include "fs2d_kernels.hpp"
@@ -54,6 +55,11 @@ static_assert(kLoopWaves > 1 + kLoaders + kPollers, "a spare wave collects |r|")
 inline bool loop_fits(const SkGeom& g, int ncu) {
     return g.S <= kLoopMaxStrips && g.nx <= kLoopMaxNx && ncu >= 8 * kLoopMaxStrips;
 }
+// Whether the strips that wait for each other, at most kLoopMaxStrips per launch
+// and one launch per hardware queue, leave half of a stream's CUs to others: on
+// 256 CUs with up to 8 queues.  The other side is separate launches with the
+// same order of the sums, so no result depends on it.
+inline bool loop_room(int cus, int queues) { return cus >= 2 * queues * kLoopMaxStrips; }
 // Device words of one simulation: kLoopWords per strip, then a tagged row per strip.
 __host__ __device__ inline size_t loop_words(const SkGeom& g) { return (size_t)g.S * (kLoopWords + 4 * g.T4); }
 

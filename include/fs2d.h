@@ -249,7 +249,10 @@ const char* fs2d_status_string(int status);
  *     iterations, whose launches size themselves to the device.
  *     Grids of at most 1024 rows and 576 columns, and ensembles of them, run
  *     the whole PCG in one launch, which uses neither pcg_grid nor fused_pcg
- *     (unless one of its phases is timed, fs2d_set_timing).
+ *     (unless one of its phases is timed, fs2d_set_timing, or its workgroups,
+ *     which wait for each other, could crowd each other out: GPU_MAX_HW_QUEUES
+ *     above 8, or a stream whose CU mask leaves it fewer than 128 CUs; then
+ *     launches per iteration give the same bits).
  *   sweep_prefetch: (ensembles) the batched triangular solves' loaders issue
  *     their first loads before testing whether their member has converged.
  *   fused_pcg: (single handles) 1, the default for solver layouts of at least

@@ -1,0 +1,36 @@
+"""The one-launch PCG's workgroups wait for each other, at most 16 per launch and
+one launch per hardware queue.  A process that asks HIP for more queues than the
+CUs have room for gets launches per iteration, with the same bits."""
+import pytest
+
+import fs2d
+from test_gpu_batch import assert_same
+from test_gpu_pcg_launches import liquid, stir
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("queues,one", [("4", True), ("8", True), ("9", False), ("16", False), ("", True)])
+def test_queues_decide_between_one_launch_and_several(queues, one, monkeypatch):
+    m = [liquid(kind, nx, ny) for kind, nx, ny in (("dam", 64, 64), ("blocks", 96, 450))]
+    plain = [fs2d.Sim(c, **kw) for c, kw in m]
+    monkeypatch.setenv("GPU_MAX_HW_QUEUES", queues)  # HIP itself has read its value before
+    sims = [fs2d.Sim(c, **kw) for c, kw in m]
+    captured = [fs2d.Sim(c, **kw) for c, kw in m]
+    batch = fs2d.Batch(m)
+    for k in range(2):
+        stir((plain[k], sims[k], captured[k], batch.sims[k]))
+        captured[k].set_graph(True)
+        sims[k].set_timing(True, only=["pcg_one_launch"])
+    batch.set_timing(True)
+    steps = 3
+    for step in range(steps):
+        batch.step()
+        for k in range(2):
+            for s in (plain[k], sims[k], captured[k]):
+                s.step()
+            for what, s in (("single", sims[k]), ("captured", captured[k]), ("member", batch.sims[k])):
+                assert_same(plain[k], s, "%s queues, step %d, %s %d" % (queues, step, what, k))
+    for x in sims + [batch]:
+        assert x.kernel_times()["pcg_one_launch"][1] == (steps if one else 0)
+    batch.close()
