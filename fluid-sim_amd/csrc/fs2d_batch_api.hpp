@@ -673,13 +673,16 @@ void bstep_stages(const fs2d_batch* B, std::vector<int>& before, std::vector<int
     }
 }
 
+// Iterations in a captured step; a solve in one launch has no such budget.
+int bgraph_budget(const fs2d_batch* B) { return bpcg_in_loop(B) ? 0 : B->graph_budget; }
+
 // `pre`: the stages before the projection, the assembly, factor and
 // graph_budget PCG iterations of every member; `post`: the pressures' copy
 // and the stages after the projection.  Captured with the batch's host flags
 // as fs2d_batch_step sets them (sort invalid at the start of a step).
 fs2d_status bcapture_step(fs2d_batch* B, fs2d_batch::Captured& G) {
     G.maps = B->d_maps;
-    G.budget = B->graph_budget;
+    G.budget = bgraph_budget(B);
     G.pcg_grid = B->pcg_grid;
     G.prefetch = B->sweep_prefetch ? 1 : 0;
     G.fused = B->fused_pcg ? 1 : 0;
@@ -723,7 +726,7 @@ fs2d_status bstep_graph(fs2d_batch* B) {
     if (B->graph_budget <= 0) bupdate_graph_budget(B, B->last_iters_hint);
     fs2d_batch::Captured* G = nullptr;
     for (auto& g : B->graphs)
-        if (g.maps == B->d_maps && g.budget == B->graph_budget && g.pcg_grid == B->pcg_grid &&
+        if (g.maps == B->d_maps && g.budget == bgraph_budget(B) && g.pcg_grid == B->pcg_grid &&
             g.prefetch == (B->sweep_prefetch ? 1 : 0) && g.fused == (B->fused_pcg ? 1 : 0))
             G = &g;
     if (!G) {
