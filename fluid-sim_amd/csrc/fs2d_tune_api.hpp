@@ -20,7 +20,9 @@
 // iterations of the projection (tolerance 0, so every member runs them all),
 // best of three after a warm-up, and keeps the fastest.  The choice is
 // recorded in a text file under a key of the device and the problem (grid
-// sizes, mode), and read from there by later calls with the same key.
+// sizes, mode), and read from there by later calls with the same key.  Where
+// the PCG is one launch no candidate differs from another, and the handle's
+// current shapes are recorded without timing any.
 
 namespace {
 
@@ -163,6 +165,11 @@ fs2d_status fs2d_autotune(fs2d_sim* s, int iters, const char* cache_path, fs2d_t
         if (out) *out = best;
         return FS2D_OK;
     }
+    if (pcg_in_loop(s)) {  // one launch whatever the choice: nothing to time
+        cache_store(cache_path, key, best);
+        if (out) *out = best;
+        return FS2D_OK;
+    }
     const double tol = s->tol;
     const int max_iters = s->max_iters, hint = s->last_iters_hint;
     s->tol = 0.0;
@@ -219,6 +226,12 @@ fs2d_status fs2d_batch_autotune(fs2d_batch* B, int iters, const char* cache_path
     if (cache_lookup(cache_path, key, &best)) {
         if (from_cache) *from_cache = 1;
         TRY(fs2d_batch_set_tuning(B, &best));
+        if (out) *out = best;
+        return FS2D_OK;
+    }
+    if (bpcg_in_loop(B)) {  // one launch whatever the choice: nothing to time
+        B->tuned = true;
+        cache_store(cache_path, key, best);
         if (out) *out = best;
         return FS2D_OK;
     }

@@ -271,7 +271,8 @@ const char* fs2d_status_string(int status);
  * projection each (tolerance 0), best of three after a warm-up; the fastest is
  * set and appended to the text file `cache_path` (NULL: none) under a key of
  * the device and the problem, from which later calls with the same key take it
- * without timing (*from_cache = 1).  Tuning overwrites the pressure and the
+ * without timing (*from_cache = 1).  Where the whole PCG is one launch, the
+ * current choice is recorded and nothing is timed.  Tuning overwrites the pressure and the
  * solver's scratch, not the state a step starts from.
  */
 typedef struct {
