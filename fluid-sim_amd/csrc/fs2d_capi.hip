@@ -41,10 +41,10 @@ const char* kKernelNames[K_COUNT] = {
 
 constexpr int kMaxBlocks = 2048;
 // Solver layouts of at least this many entries (a 512^2 grid has 294912) run
-// a PCG iteration as two launches by default: measured per iteration against
-// four launches, 0.94-0.98x from 512^2 up, 1.03-1.08x at 64^2-384^2, where
-// the separate SpMV and axpy are short and the fused launches' head and tail
-// cost more than they hide.
+// a PCG iteration as two launches by default, where the whole PCG is not one:
+// measured per iteration against four launches, 0.94-0.98x from 512^2 up,
+// 1.03-1.08x at 64^2-384^2, where the separate SpMV and axpy are short and the
+// fused launches' head and tail cost more than they hide.
 constexpr long kFusedPcgMinEntries = 1L << 18;
 
 int blocks_for(long n) {

@@ -182,8 +182,8 @@ __device__ __forceinline__ double loop_block_sum(double acc, double* part) {
 }
 
 // The SpMV alone, a strip per workgroup, with the partial w.s of each strip:
-// what the loop computes, for the separate launches that per-kernel timing and
-// batches with larger members need.  s' of the neighbouring rows is formed from
+// what the loop computes, for the separate launches that timing their phases,
+// batches with larger members and streams without room for the loop need.  s' of the neighbouring rows is formed from
 // their own s and z; outside the active range s' and w are set to zero, for the
 // p/r update's launch, which covers the whole array.
 __device__ __forceinline__ void spmv_strip_body(const SkGeom& g, const float* __restrict__ Adiag,

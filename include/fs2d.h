@@ -213,7 +213,9 @@ fs2d_status fs2d_max_velocity(fs2d_sim* sim, double* out);
  * the previous solve's iteration count; a step is captured again when a
  * parameter, the particle count, the budget or a buffer it uses changed (at
  * most four captures are kept).  Results are bit-identical to the uncaptured
- * step.  Timing (fs2d_set_timing) runs uncaptured steps. */
+ * step.  Where the whole solve is one launch (see fs2d_tuning) the first graph
+ * holds all of it: no budget, no check between the graphs.  Timing
+ * (fs2d_set_timing) runs uncaptured steps. */
 fs2d_status fs2d_set_graph(fs2d_sim* sim, int enable);
 
 /* Per-kernel timing with HIP events on the handle's stream (no reference
@@ -257,8 +259,9 @@ const char* fs2d_status_string(int status);
  *     their first loads before testing whether their member has converged.
  *   fused_pcg: (single handles) 1, the default for solver layouts of at least
  *     2^18 entries (ceil(size_y / 64) * 64 * ceil((size_x + 64) / 32) * 32;
- *     512 x 512 has 294912; below it the separate launches measured 3-8%
- *     faster): a PCG iteration is two launches instead of four: the p/r update with the forward solve, whose
+ *     700 x 320 has 245760 and 700 x 384 has 294912; below 2^18 the separate
+ *     launches measured 3-8% faster): a PCG iteration of a grid past the one
+ *     launch is two launches instead of four: the p/r update with the forward solve, whose
  *     strips start as soon as the update has passed them, and the backward
  *     solve with the next iteration's SpMV, whose workgroups take each region
  *     as soon as the solve's strips around it have finished (the stopping
@@ -299,9 +302,9 @@ fs2d_status fs2d_autotune(fs2d_sim* sim, int iters, const char* cache_path, fs2d
  * <= 524288 (512 x 512 does, 700 x 700 does not).  Larger grids are rejected
  * with FS2D_ERR_ARG before any device work.  Calls on one GPU share that
  * buffer: calls that overlap on one GPU (two threads, or two streams) race.
- * The call returns after the solve has finished on `stream`; the host reads
- * the convergence flag between chunks of iterations with synchronising
- * copies into its own stack.  Failures are explained by fs2d_last_error(NULL).
+ * The call returns after the solve has finished on `stream`; where the solve is
+ * by launches per iteration, the host reads the convergence flag between chunks
+ * of iterations with synchronising copies into its own stack.  Failures are explained by fs2d_last_error(NULL).
  */
 typedef struct {
     int size_x;
